@@ -111,16 +111,20 @@ typedef struct msfem_solver_opts {
                                  by later calls with the same batch layout, pointers and
                                  options (msfem_ctx_profile is not updated; time it with
                                  msfem_ctx_mark) */
-  int32_t coarse_space;       /* 1 (default): two-level preconditioner (Jacobi plus the
-                                 bilinear coarse space of an 8 x 8 coarse grid per local
-                                 problem, solved exactly) for the 64^2 and 128^2 classes at
-                                 the default launch shapes; on 64^2 classes also the
-                                 intermediate hat levels of spacing 2 and 4, on FP32 128^2
-                                 classes those of spacing 4 and 8, scaled by their diagonals
-                                 (additive);
-                                 2: the two-level form without the
-                                 intermediate levels; 0: Jacobi only.  Same converged
-                                 values, fewer iterations. */
+  int32_t coarse_space;       /* 1 (default): 2D classes of 9..128 fine cells per side are
+                                 solved directly (FP64 nested dissection, then the residual
+                                 test below and, where it fails, one correction) unless x0 or
+                                 a launch shape is given; 64^2 classes only in FP64 and from
+                                 32 cells.  Other 64^2 and 128^2 classes run CG with the
+                                 two-level preconditioner (Jacobi plus the bilinear coarse
+                                 space of an 8 x 8 coarse grid per local problem, solved
+                                 exactly) at the default launch shapes; on 64^2 classes also
+                                 the intermediate hat levels of spacing 2 and 4, on FP32
+                                 128^2 classes those of spacing 4 and 8, scaled by their
+                                 diagonals (additive);
+                                 2: CG with the two-level form without the
+                                 intermediate levels; 0: CG with Jacobi only.  Same
+                                 converged values, fewer iterations. */
   int32_t q1_start;           /* without x0: 1 (default) = the interior starts at the Q1
                                  interpolant of the Dirichlet data (box cells: the nodal
                                  Q1 function itself; general cells: the transfinite
@@ -172,7 +176,8 @@ typedef struct msfem_batch_out {
   double *Ae;       /* [n_cells][nb][nb]  A^K_ij = phi_i^T K phi_j */
   double *Fe;       /* [n_cells][nb]      F^K_i  = phi_i^T b       */
   double *bases;    /* optional (NULL): [sum_c nb (nf_c+1)^dim] basis nodal values */
-  int32_t *iters;   /* optional: [n_cells][nb] inner CG iterations */
+  int32_t *iters;   /* optional: [n_cells][nb] inner CG iterations; direct solves: 1, 2 with
+                       a correction, 0 where the start already met the tolerance */
   int32_t *status;  /* optional: [n_cells][nb] 0 converged, 1 not converged */
   double *resid;    /* optional: [n_cells][nb] final true residual norm */
   double *energy_bound; /* optional: [n_cells][nb] a posteriori bound of the relative
@@ -190,7 +195,7 @@ int msfem_ctx_destroy(msfem_ctx *ctx);
 const char *msfem_last_error(const msfem_ctx *ctx); /* ctx may be NULL (creation errors) */
 void msfem_default_opts(msfem_solver_opts *opts);
 /* 1 if a class of nf fine cells per side with these options, coefficient kind
- * and geometry (general: vertex cells) runs the two-level local solve on this
+ * and geometry (general: vertex cells) runs the two-level form when it is solved by CG on this
  * context (its launch-shape table applied), 2 if its preconditioner also takes
  * the intermediate hat levels (spacing 2 and 4 at 64^2, 4 and 8 at 128^2), else
  * 0.  No counterpart in the

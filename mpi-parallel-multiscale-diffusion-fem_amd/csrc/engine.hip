@@ -74,6 +74,9 @@ struct msfem_ctx {
   hipEvent_t scratch_done = nullptr;
   hipStream_t scratch_stream = nullptr;
   bool scratch_recorded = false;
+  // direct solves: the plan of every resolution met so far and its device tables (never
+  // rewritten, so builds in flight and captured graphs may hold them)
+  std::map<int, std::pair<DirectHost, void *>> direct;
   // the current build computes the energy terms (stopping rule or bound), and
   // whether its last basis comes from the partition of unity
   bool energy_terms = false;
@@ -442,6 +445,52 @@ int class_variant(msfem_ctx *ctx, const msfem_batch *in, const msfem_solver_opts
   return variant;
 }
 
+// Whether size class k runs the direct solves: box cells and quadrilaterals of 9..128 fine cells
+// per side at the default options.  A caller's x0, an explicit launch shape or another
+// coarse_space asks for the iterative solve.  64^2 cells in FP32 keep it too (4096 cells: 5.0 ms
+// against 8.9 ms direct), and so do classes of fewer than 32 cells of 64^2: those are what
+// callers compare starts, preconditioners and iteration counts on.
+constexpr int kDirect64Cells = 32;
+bool class_direct(const Plan &p, const msfem_batch *in, const msfem_solver_opts *o, size_t k)
+{
+  const int nf = p.class_nf[k];
+  if (!direct_supported(in->dim, nf) || in->x0 || o->coarse_space != 1 || o->variant != 0)
+    return false;
+  return nf != 64 || (o->precision == MSFEM_PREC_FP64 && (int)p.class_cells[k].size() >= kDirect64Cells);
+}
+
+// Doubles of the direct classes' scratch before size class k_end (each class owns a slice).
+size_t direct_doubles(msfem_ctx *ctx, const msfem_batch *in, const msfem_solver_opts *o, size_t k_end)
+{
+  const Plan &p = ctx->plan;
+  size_t n = 0;
+  for (size_t k = 0; k < k_end && k < p.class_nf.size(); ++k)
+    if (class_direct(p, in, o, k))
+      n += direct_scratch_doubles(ctx->direct.at(p.class_nf[k]).first, (int)p.class_cells[k].size(), in->coef_kind,
+                                  in->vertices != nullptr);
+  return n;
+}
+
+// The direct plan of resolution nf in ctx->direct.
+int need_direct_plan(msfem_ctx *ctx, int nf)
+{
+  if (ctx->direct.count(nf))
+    return MSFEM_OK;
+  DirectHost h;
+  std::vector<char> blob;
+  direct_host_plan(nf, h, blob);
+  void *d = nullptr;
+  HIP_TRY(ctx, hipMalloc(&d, blob.size()));
+  const hipError_t e = hipMemcpy(d, blob.data(), blob.size(), hipMemcpyHostToDevice);
+  if (e != hipSuccess)
+    {
+      hipFree(d);
+      return fail(ctx, MSFEM_ERR_HIP, "hipMemcpy (direct plan): %s", hipGetErrorString(e));
+    }
+  ctx->direct[nf] = {h, d};
+  return MSFEM_OK;
+}
+
 // Whether size class nf runs the two-level local solve.
 bool class_coarse(msfem_ctx *ctx, const msfem_batch *in, const msfem_solver_opts *o, int nf)
 {
@@ -466,7 +515,7 @@ size_t ml_floats(msfem_ctx *ctx, const msfem_batch *in, const msfem_solver_opts 
   const Plan &p = ctx->plan;
   size_t n = 0;
   for (size_t k = 0; k < k_end && k < p.class_nf.size(); ++k)
-    if (class_ml(ctx, in, o, p.class_nf[k]))
+    if (!class_direct(p, in, o, k) && class_ml(ctx, in, o, p.class_nf[k]))
       n += p.class_cells[k].size() * (size_t)kMlFloats;
   return n;
 }
@@ -478,7 +527,7 @@ size_t coarse_inv_doubles(msfem_ctx *ctx, const msfem_batch *in, const msfem_sol
   const Plan &p = ctx->plan;
   size_t n = 0;
   for (size_t k = 0; k < k_end && k < p.class_nf.size(); ++k)
-    if (class_coarse(ctx, in, o, p.class_nf[k]))
+    if (!class_direct(p, in, o, k) && class_coarse(ctx, in, o, p.class_nf[k]))
       n += p.class_cells[k].size() * (size_t)kCoarseDofs * kCoarseDofs;
   return n;
 }
@@ -493,7 +542,7 @@ size_t stream_work_doubles(msfem_ctx *ctx, const msfem_batch *in, const msfem_so
   if (o->precision != MSFEM_PREC_FP64)
     return 0;
   for (size_t k = 0; k < k_end && k < p.class_nf.size(); ++k)
-    if (build_mode(in, p.class_nf[k]) == kModeStream)
+    if (!class_direct(p, in, o, k) && build_mode(in, p.class_nf[k]) == kModeStream)
       n += p.class_cells[k].size() * (size_t)(o->partition_of_unity ? p.nb - 1 : p.nb) *
            stream_q_slots(p.class_nf[k]);
   return n;
@@ -505,7 +554,7 @@ size_t generic_work_total(msfem_ctx *ctx, const msfem_batch *in, const msfem_sol
   const Plan &p = ctx->plan;
   size_t n = 0;
   for (size_t k = 0; k < k_end && k < p.class_nf.size(); ++k)
-    if (build_mode(in, p.class_nf[k]) == kModeGeneric)
+    if (!class_direct(p, in, o, k) && build_mode(in, p.class_nf[k]) == kModeGeneric)
       n += p.class_cells[k].size() * (size_t)(o->partition_of_unity ? p.nb - 1 : p.nb) *
            generic_work_doubles(in->dim, p.class_nf[k]);
   return n;
@@ -522,20 +571,21 @@ int launch_class_prepare(msfem_ctx *ctx, const msfem_batch *in, const msfem_solv
   const int *cells = d_cells(ctx) + p.cells_dev_off[k];
   const bool fp32 = o->precision == MSFEM_PREC_FP32_REFINE;
   const int mode = build_mode(in, nf);
-  if (mode == kModeGlobal)
+  const bool direct = class_direct(p, in, o, k); // (forms the fine cells itself)
+  if (!direct && mode == kModeGlobal)
     HIP_TRY(ctx, launch_prep_cond_2d(ncls, cells, nf, in->coef_kind, in->box, in->vertices, in->coef, d_off(ctx, 0),
                                      cond, d_off(ctx, 2), st));
-  if (mode == kModeStream)
+  if (!direct && mode == kModeStream)
     HIP_TRY(ctx, launch_prep_couplings_2d(ncls, cells, nf, in->coef_kind, in->box, in->vertices, in->coef,
                                           d_off(ctx, 0), cond, d_off(ctx, 2), fp32, st));
-  if (mode == kModeGeneric)
+  if (!direct && mode == kModeGeneric)
     HIP_TRY(ctx, launch_generic_prep(in->dim, ncls, cells, nf, in->coef_kind, in->box, in->vertices, in->coef,
                                      d_off(ctx, 0), cond, d_off(ctx, 2), st));
   if (in->vertices && in->dim == 2) // the solve kernels read the boundary data from the bases
     HIP_TRY(ctx, launch_quad_dirichlet_2d(ncls, cells, nf, in->vertices, bases, d_off(ctx, 1), st));
   else if (in->vertices)
     HIP_TRY(ctx, launch_hex_dirichlet_3d(ncls, cells, nf, in->vertices, bases, d_off(ctx, 1), st));
-  if (class_coarse(ctx, in, o, nf))
+  if (!direct && class_coarse(ctx, in, o, nf))
     {
       double *base = (double *)ctx->bufs["coarse_inv"].p;
       if (!base)
@@ -543,7 +593,7 @@ int launch_class_prepare(msfem_ctx *ctx, const msfem_batch *in, const msfem_solv
       HIP_TRY(ctx, launch_coarse_setup_2d(ncls, cells, nf, in->coef_kind, in->box, in->vertices, in->coef,
                                           d_off(ctx, 0), base + coarse_inv_doubles(ctx, in, o, k), st));
     }
-  if (class_ml(ctx, in, o, nf))
+  if (!direct && class_ml(ctx, in, o, nf))
     {
       float *mb = (float *)ctx->bufs["ml_inv"].p;
       if (!mb)
@@ -598,13 +648,20 @@ int launch_class_solve(msfem_ctx *ctx, const msfem_batch *in, const msfem_solver
   a.max_refine = o->max_refine;
   a.ptol = o->energy_tol > 0 ? (const double *)ctx->bufs["ptol"].p : nullptr;
   const int variant = class_variant(ctx, in, o, nf);
+  const bool direct = class_direct(p, in, o, k);
   a.cinv = nullptr;
-  if (class_coarse(ctx, in, o, nf))
+  if (!direct && class_coarse(ctx, in, o, nf))
     a.cinv = (const double *)ctx->bufs["coarse_inv"].p + coarse_inv_doubles(ctx, in, o, k);
   a.mlinv = nullptr;
-  if (class_ml(ctx, in, o, nf))
+  if (!direct && class_ml(ctx, in, o, nf))
     a.mlinv = (const float *)ctx->bufs["ml_inv"].p + ml_floats(ctx, in, o, k);
-  if (mode == kModeGeneric)
+  if (direct)
+    {
+      const auto &d = ctx->direct.at(nf);
+      double *ds = (double *)ctx->bufs["direct"].p + direct_doubles(ctx, in, o, k);
+      HIP_TRY(ctx, launch_direct_solve(d.first, (const char *)d.second, a, ncls, in->coef_kind, ds, st));
+    }
+  else if (mode == kModeGeneric)
     {
       double *gw = (double *)ctx->bufs["gen_work"].p;
       if (!gw)
@@ -801,6 +858,18 @@ int enqueue_build(msfem_ctx *ctx, const msfem_batch *in, const msfem_solver_opts
   if (p.cond_total > 0)
     {
       rc = scratch(ctx, "cond", p.cond_total * sizeof(double), (void **)&cond);
+      if (rc)
+        return rc;
+    }
+  // plans and factor scratch of the direct classes (made before any capture)
+  for (size_t k = 0; k < p.class_nf.size(); ++k)
+    if (class_direct(p, in, o, k) && (rc = need_direct_plan(ctx, p.class_nf[k])))
+      return rc;
+  const size_t dir_doubles = direct_doubles(ctx, in, o, p.class_nf.size());
+  if (dir_doubles > 0)
+    {
+      void *d;
+      rc = scratch(ctx, "direct", dir_doubles * sizeof(double), &d);
       if (rc)
         return rc;
     }
@@ -1211,6 +1280,8 @@ int msfem_ctx_destroy(msfem_ctx *ctx)
   for (auto &kv : ctx->bufs)
     if (kv.second.p)
       hipFree(kv.second.p);
+  for (auto &kv : ctx->direct)
+    hipFree(kv.second.second);
   if (ctx->stream)
     hipStreamDestroy(ctx->stream);
   delete ctx;

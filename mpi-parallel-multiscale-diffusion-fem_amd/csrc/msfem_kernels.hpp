@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 #include "msfem_device.hpp"
 
 namespace msfem {
@@ -37,6 +39,54 @@ hipError_t launch_quad_dirichlet_2d(int n_cells_class, const int *cells, int nf,
 // local3d.hip
 int local3d_variants(int nf);
 hipError_t launch_local_solve_3d(bool fp32, int nf, int variant, const LocalArgs &a, hipStream_t st);
+
+// direct.hip: the direct local solves in 2D (nested dissection, FP64).
+struct DirectFront;
+struct DirectLeaf;
+struct DirectLeafType;
+constexpr int kDirectLevels = 4; // front levels of the largest resolution
+// What the host keeps of a resolution's plan (direct_plan.hpp); the tables are in device memory.
+struct DirectHost {
+  int nf, depth;
+  int n_fronts[kDirectLevels], max_rows[kDirectLevels], max_elim[kDirectLevels];
+  size_t fronts_at[kDirectLevels], leaves_at, types_at, tables_at; // byte offsets in the device tables
+  long long cell_doubles;                                          // factor scratch of one cell
+};
+struct DirectArgs {
+  int nf, depth, level, nb, nb_solve, coef_kind, q1_start;
+  int second;                     // 1: the correction pass (unknown = a.corr, right-hand side = a.loads)
+  int n_fronts[kDirectLevels];
+  const DirectFront *fronts[kDirectLevels];
+  const DirectLeaf *leaves;
+  const DirectLeafType *types;
+  const uint32_t *tables;
+  const int *cells;               // batch cells of this chunk, one per slot
+  const double *box, *verts, *coef;
+  const long long *coef_off, *bas_off;
+  double *bases;
+  double *scratch;                // [slot][cell_doubles]
+  long long cell_doubles;
+  const int *need;                // correction pass: cells to work on; nullptr = all
+  const double *loads;            // correction pass: residuals [slot][4][nodes]
+  double *loads_out, *corr;       // [slot][4][nodes]
+  double *cond;                   // stored fine cells: conductances [slot][6][nf^2]
+  double *part;                   // residual sums [slot][task][12]
+  int *need_out;                  // [slot]
+  const double *ptol;
+  double rel_tol, abs_tol;
+  int *iters, *status;
+  double *resid;
+  // the pass's unknown: bases, or the corrections
+  __device__ double *x_of(int slot, int cell) const
+  {
+    return second ? corr + (size_t)slot * 4 * (nf + 1) * (nf + 1) : bases + bas_off[cell];
+  }
+};
+bool direct_supported(int dim, int nf);
+void direct_host_plan(int nf, DirectHost &h, std::vector<char> &blob);
+size_t direct_scratch_doubles(const DirectHost &h, int n_cells, int coef_kind, bool general);
+hipError_t launch_direct_solve(const DirectHost &h, const char *blob, const LocalArgs &in, int n_cells, int coef_kind,
+                               double *scratch, hipStream_t st);
 
 // generic.hip: the local solve for resolutions and coefficient kinds outside the
 // tuned kernels.  Element matrices [nf^d][2^d][2^d] per cell (offsets elem_off,
