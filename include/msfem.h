@@ -316,9 +316,11 @@ int msfem_coarse_solve_device(msfem_ctx *ctx, int dim, int nc, const double *Kc,
  * tight serving loops, harnesses that forbid hipMalloc).  The kernels of
  * msfem_coarse_solve_device run with their scratch in a fixed 16 MiB device
  * array of the library (one per GPU, held until the process ends, its address
- * looked up when a context is created on that GPU); the call enqueues one
- * kernel on `stream` and calls no hipMalloc, hipFree or other allocating
- * routine.  Systems whose scratch exceeds the array (for power-of-two sizes:
+ * looked up when a context is created on that GPU); the call only enqueues
+ * kernels on `stream` and calls no hipMalloc, hipFree or other allocating
+ * routine.  Systems whose multigrid scratch exceeds the array run the Jacobi-CG
+ * if its smaller scratch fits and their size does not halve evenly to a small
+ * grid.  Other systems whose scratch exceeds the array (for power-of-two sizes:
  * 2D beyond 256 x 256 cells, 3D beyond 32^3) are rejected with MSFEM_ERR_ARG.  Every call on one
  * GPU shares that GPU's array, so calls that overlap on one GPU (different
  * streams, no ordering between them) race; the kernels write every scratch
@@ -344,7 +346,8 @@ int msfem_reconstruct_device(msfem_ctx *ctx, int dim, int n_cells, const int32_t
  * beside the MsFEM (source/main.cxx:33-35).  Q1 on the n x n fine mesh of the
  * unit square with the coefficient tile `coef` (host; one cell of nf = n in
  * the batch layout of coef_kind), load f (rhs_kind, rhs_value) and boundary
- * data bc_kind (MSFEM_BC_*); FP64 Jacobi-PCG over many workgroups, stopped at
+ * data bc_kind (MSFEM_BC_*); FP64 CG preconditioned with a multigrid V-cycle
+ * over many workgroups, stopped at
  * ||r||_2 <= rel_tol ||r_0||_2 (r_0: residual of the Dirichlet lift) or
  * max_iter iterations (then MSFEM_ERR_NOCONV, u still written).  u: host
  * [(n+1)^2] nodal values, lexicographic; 2D only (dim = 2). */

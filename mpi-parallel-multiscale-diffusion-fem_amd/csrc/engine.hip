@@ -1474,7 +1474,7 @@ int msfem_coarse_solve_device(msfem_ctx *ctx, int dim, int nc, const double *Kc,
   if (rc)
     return rc;
   HIP_TRY(ctx, launch_coarse_solve(dim, nc, Kc, Fc, cmask, cval, rel_tol, max_iter, u, iters, work,
-                                   (hipStream_t)stream));
+                                   coarse_solve_work_doubles(dim, nc), (hipStream_t)stream));
   return retire_scratch(ctx, (hipStream_t)stream, capturing);
 }
 
@@ -1490,7 +1490,7 @@ int msfem_coarse_solve_device_noalloc(msfem_ctx *ctx, int dim, int nc, const dou
   if ((dim == 2 && nc > 4096) || (dim == 3 && nc > 256))
     return fail(ctx, MSFEM_ERR_ARG, "coarse system of %d^%d cells exceeds the fixed scratch of %zu bytes", nc, dim,
                 noalloc_scratch_bytes());
-  const size_t need = coarse_solve_work_doubles(dim, nc) * sizeof(double);
+  const size_t need = coarse_solve_least_doubles(dim, nc) * sizeof(double);
   if (need > noalloc_scratch_bytes())
     return fail(ctx, MSFEM_ERR_ARG,
                 "coarse system of %d^%d cells needs %zu bytes of scratch, more than the fixed %zu of the "
@@ -1505,7 +1505,8 @@ int msfem_coarse_solve_device_noalloc(msfem_ctx *ctx, int dim, int nc, const dou
     }
   if (!w)
     return fail(ctx, MSFEM_ERR_HIP, "fixed scratch of device %d unavailable", ctx->device);
-  HIP_TRY(ctx, launch_coarse_solve(dim, nc, Kc, Fc, cmask, cval, rel_tol, max_iter, u, iters, w, (hipStream_t)stream));
+  HIP_TRY(ctx, launch_coarse_solve(dim, nc, Kc, Fc, cmask, cval, rel_tol, max_iter, u, iters, w,
+                                   noalloc_scratch_bytes() / sizeof(double), (hipStream_t)stream));
   return MSFEM_OK;
 }
 
@@ -1616,67 +1617,59 @@ int msfem_fine_solve(msfem_ctx *ctx, int dim, int n, int coef_kind, const double
   double *Kc = s.alloc<double>("f_Kc", nn * 9, true), *Fc = s.alloc<double>("f_Fc", nn, true);
   unsigned char *cm = s.alloc<unsigned char>("f_cm", nn, true);
   double *cv = s.alloc<double>("f_cv", nn, true);
-  double *vec = s.alloc<double>("f_vec", 5 * nn, true);
-  double *part = s.alloc<double>("f_part", 2 * (size_t)fine_cg_blocks((int)nn), true);
-  FineCgState *state = s.alloc<FineCgState>("f_state", 1, true);
+  const MgLayout g = mg_layout(2, n);
+  double *w = s.alloc<double>("f_mg", (size_t)g.total, true), *du = s.alloc<double>("f_u", nn, true);
+  int *dit = s.alloc<int>("f_it", 1, true);
   if (s.rc)
     return s.rc;
   HIP_TRY(ctx, launch_fine_elements_2d(n, coef_kind, dcoef, rhs_kind, rhs_value, Ae, Fe, st));
   HIP_TRY(ctx, launch_coarse_assemble(2, n, Ae, Fe, bc_kind, Kc, Fc, cm, cv, st));
-  FineCgState init = {};
-  init.rel_tol = rel_tol;
-  init.max_iter = max_iter;
-  HIP_TRY(ctx, hipMemcpyAsync(state, &init, sizeof init, hipMemcpyHostToDevice, st));
-  FineCgArgs a;
-  a.dim = 2;
-  a.np = (int)np;
-  a.nn = (int)nn;
-  a.Kc = Kc;
-  a.Fc = Fc;
-  a.cmask = cm;
-  a.cval = cv;
-  a.x = vec;
-  a.r = vec + nn;
-  a.p = vec + 2 * nn;
-  a.q = vec + 3 * nn;
-  a.dinv = vec + 4 * nn;
-  a.part = part;
-  a.state = state;
-  HIP_TRY(ctx, launch_fine_cg_start(a, st));
-  // CG steps in blocks of kSteps, captured once as a graph and replayed until
-  // the device-side state says done (finished steps turn into no-ops)
-  constexpr int kSteps = 32;
-  hipGraph_t g = nullptr;
-  hipGraphExec_t x = nullptr;
-  HIP_TRY(ctx, hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  const hipError_t el = launch_fine_cg_steps(a, kSteps, st);
-  const hipError_t ec = hipStreamEndCapture(st, &g);
-  if (el != hipSuccess || ec != hipSuccess)
+  HIP_TRY(ctx, launch_mg_setup(2, g, Kc, Fc, cm, cv, rel_tol, max_iter, w, st));
+  const double *x = w + g.off_cx;
+  MgState host = {};
+  hipError_t e = hipSuccess;
+  if (g.tail == 0)
     {
-      if (g)
-        hipGraphDestroy(g);
-      return fail(ctx, MSFEM_ERR_HIP, "fine CG capture: %s", hipGetErrorString(el != hipSuccess ? el : ec));
-    }
-  hipError_t e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-  hipGraphDestroy(g);
-  if (e != hipSuccess)
-    return fail(ctx, MSFEM_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
-  FineCgState host = {};
-  for (int done_steps = 0;; done_steps += kSteps)
-    {
-      e = hipMemcpyAsync(&host, state, sizeof host, hipMemcpyDeviceToHost, st);
+      HIP_TRY(ctx, launch_mg_small(2, g, Kc, du, dit, w, st));
+      x = du;
+      e = hipMemcpyAsync(&host, w + g.off_state, sizeof host, hipMemcpyDeviceToHost, st);
       if (e == hipSuccess)
         e = hipStreamSynchronize(st);
-      if (e != hipSuccess || host.done || done_steps > max_iter)
-        break;
-      e = hipGraphLaunch(x, st);
-      if (e != hipSuccess)
-        break;
     }
-  hipGraphExecDestroy(x);
+  else
+    {
+      // CG iterations in blocks of kSteps, captured once as a graph and replayed
+      // until the device-side state says done (finished ones turn into no-ops)
+      constexpr int kSteps = 8;
+      hipGraph_t gr = nullptr;
+      hipGraphExec_t gx = nullptr;
+      HIP_TRY(ctx, hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+      const hipError_t el = launch_mg_iterations(2, g, kSteps, Kc, w, st);
+      const hipError_t ec = hipStreamEndCapture(st, &gr);
+      if (el != hipSuccess || ec != hipSuccess)
+        {
+          if (gr)
+            hipGraphDestroy(gr);
+          return fail(ctx, MSFEM_ERR_HIP, "fine CG capture: %s", hipGetErrorString(el != hipSuccess ? el : ec));
+        }
+      e = hipGraphInstantiate(&gx, gr, nullptr, nullptr, 0);
+      hipGraphDestroy(gr);
+      if (e != hipSuccess)
+        return fail(ctx, MSFEM_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
+      do
+        {
+          e = hipGraphLaunch(gx, st);
+          if (e == hipSuccess)
+            e = hipMemcpyAsync(&host, w + g.off_state, sizeof host, hipMemcpyDeviceToHost, st);
+          if (e == hipSuccess)
+            e = hipStreamSynchronize(st);
+        }
+      while (e == hipSuccess && !host.done);
+      hipGraphExecDestroy(gx);
+    }
   if (e != hipSuccess)
     return fail(ctx, MSFEM_ERR_HIP, "fine CG: %s", hipGetErrorString(e));
-  HIP_TRY(ctx, hipMemcpyAsync(u, a.x, nn * sizeof(double), hipMemcpyDeviceToHost, st));
+  HIP_TRY(ctx, hipMemcpyAsync(u, x, nn * sizeof(double), hipMemcpyDeviceToHost, st));
   HIP_TRY(ctx, hipStreamSynchronize(st));
   if (iters)
     *iters = host.iters;

@@ -138,28 +138,39 @@ hipError_t launch_energy_bound(int n_cells_class, const int *cells, int nb, int 
 hipError_t launch_sub(size_t n, const double *x, const double *y, double *d, hipStream_t st);
 hipError_t launch_energy_ratio(int n_cells, int nb, const double *Ad, const double *Ar, double *err, hipStream_t st);
 
-// coarse.hip
-// Scratch layout of the multigrid-preconditioned coarse CG (offsets in doubles).
-constexpr int kMgMaxLevels = 12;
-constexpr int kMgMaxDense = 343; // largest coarsest level solved densely (7^3 or 18^2 nodes)
+// mg.hip: multigrid-preconditioned CG on structured stencil matrices.
+// Scratch layout (offsets in doubles).
+constexpr int kMgMaxLevels = 15;
 struct MgLayout {
-  int levels;                        // 0: no multigrid for this size (Jacobi-PCG instead)
-  int n[kMgMaxLevels];               // cells per side of level l (n[0] = nc)
+  int levels, tail;                  // levels; the first of those that one workgroup keeps in LDS
+  int n[kMgMaxLevels];               // cells per side of level l (n[0] = nc, n[l + 1] = ceil(n[l] / 2))
   long long nn[kMgMaxLevels];        // nodes of level l
-  long long off_x[kMgMaxLevels], off_t[kMgMaxLevels], off_d[kMgMaxLevels], off_b[kMgMaxLevels],
-    off_A[kMgMaxLevels], off_u[kMgMaxLevels];
-  long long off_mask[kMgMaxLevels];  // level l >= 1: constrained-node flags, bytes at (char *)(w + off_mask[l])
-  long long off_cx, off_cr, off_cp, off_cq; // CG vectors on level 0
-  long long off_dense, off_dmap;     // coarsest Cholesky factor [F][F], free-node numbers
+  long long off_x[kMgMaxLevels], off_t[kMgMaxLevels], off_d[kMgMaxLevels], off_b[kMgMaxLevels], off_A[kMgMaxLevels];
+  long long off_cx, off_cr, off_r1, off_cp, off_p1, off_cq; // CG vectors on level 0 (r and p twice)
+  long long off_part, off_inv, off_state; // partial sums, inverse of the coarsest matrix, MgState
   long long total;
 };
+struct MgState {
+  double rz[2], rnorm, tol, rel_tol;
+  int iters, max_iter, done, converged, begun, parts_dir;
+};
 MgLayout mg_layout(int dim, int nc);
+// Galerkin levels, x = Dirichlet values, residual, state; then blocks of an even number of
+// iterations until the state says done (iterations past that end at once).  The solution is at
+// w + off_cx.  launch_mg_small: the whole iteration of a system with g.tail == 0.
+hipError_t launch_mg_setup(int dim, const MgLayout &g, const double *Kc, const double *Fc, const unsigned char *cmask,
+                           const double *cval, double rel_tol, int max_iter, double *w, hipStream_t st);
+hipError_t launch_mg_iterations(int dim, const MgLayout &g, int count, const double *Kc, double *w, hipStream_t st);
+hipError_t launch_mg_small(int dim, const MgLayout &g, const double *Kc, double *u, int *iters, double *w, hipStream_t st);
+
+// coarse.hip
 hipError_t launch_coarse_assemble(int dim, int nc, const double *Ae, const double *Fe, int bc_kind, double *Kc,
                                   double *Fc, unsigned char *cmask, double *cval, hipStream_t st);
 hipError_t launch_coarse_solve(int dim, int nc, const double *Kc, const double *Fc, const unsigned char *cmask,
                                const double *cval, double rel_tol, int max_iter, double *u, int *iters,
-                               double *work, hipStream_t st);
-size_t coarse_solve_work_doubles(int dim, int nc);
+                               double *work, size_t work_doubles, hipStream_t st);
+size_t coarse_solve_work_doubles(int dim, int nc);  // scratch of the coarse solve
+size_t coarse_solve_least_doubles(int dim, int nc); // the least it runs with
 hipError_t launch_reconstruct(int n_cells, int nb, const long long *bas_off, const long long *out_off,
                               const int *n_nodes, const double *bases, const double *w, double *u, hipStream_t st);
 
@@ -170,24 +181,8 @@ hipError_t noalloc_register_device(int device);
 double *noalloc_scratch(int device);
 size_t noalloc_scratch_bytes();
 
-// fine.hip: fine-scale standard FEM (element matrices + multi-workgroup FP64 CG
-// on a structured stencil matrix, scalars in device memory).
-struct FineCgState {
-  double rz, alpha, beta, rnorm, tol, rel_tol;
-  int iters, max_iter, done, converged;
-};
-struct FineCgArgs {
-  int dim, np, nn;
-  const double *Kc, *Fc;
-  const unsigned char *cmask;
-  const double *cval;
-  double *x, *r, *p, *q, *dinv, *part; // part: 2 * fine_cg_blocks(nn) doubles
-  FineCgState *state;
-};
-int fine_cg_blocks(int nn);
+// fine.hip: fine-scale standard FEM (element matrices and loads).
 hipError_t launch_fine_elements_2d(int n, int coef_kind, const double *coef, int rhs_kind, double rhs_value,
                                    double *Ae, double *Fe, hipStream_t st);
-hipError_t launch_fine_cg_start(const FineCgArgs &a, hipStream_t st);
-hipError_t launch_fine_cg_steps(const FineCgArgs &a, int steps, hipStream_t st);
 
 } // namespace msfem

@@ -2,7 +2,7 @@
 // callers that cannot allocate device memory (code under HIP graph capture,
 // tight serving loops, harnesses that forbid hipMalloc).  It runs the same
 // kernels as msfem_coarse_solve_device (the multigrid-preconditioned CG, or
-// Jacobi-PCG for sizes that do not coarsen) with their scratch in a fixed
+// Jacobi-CG where only its scratch fits) with their scratch in a fixed
 // device array instead of context-owned memory.
 //
 // `scratch` is a file-scope device array of kNoAllocScratchBytes (16 MiB); each
