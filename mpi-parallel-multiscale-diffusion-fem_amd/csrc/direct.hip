@@ -150,10 +150,10 @@ __device__ __forceinline__ void neg_inverse_column(const double *D, int nv, int 
 
 // Single-wave form: lower tiles (i, j) of a TILES x TILES front in acc, row by row, at most MAXE
 // eliminated rows (the pivot loop is unrolled, so a step touches exactly the tiles it needs).
-// P: LDS, 16 TILES x 4.  STORE: row r > p of W = A D^-1 at W[r * ldw + p].
+// P: LDS, 16 TILES x 4.  STORE: row r > p of W = A D^-1 at W[r (r + 1) / 2 + p].
 template <int TILES, int MAXE, bool STORE>
 __device__ __forceinline__ void eliminate_wave(d4 (&acc)[TILES * (TILES + 1) / 2], int ne, int m, double *P, double *W,
-                                               int ldw, int lane)
+                                               int lane)
 {
   const int l16 = lane & 15, kk = lane >> 4;
 #pragma unroll
@@ -183,7 +183,7 @@ __device__ __forceinline__ void eliminate_wave(d4 (&acc)[TILES * (TILES + 1) / 2
             {
               const int r = 16 * i + l16;
               if (r >= p0 + nv && r < m && kk < nv)
-                W[r * ldw + p0 + kk] = -w[i];
+                W[r * (r + 1) / 2 + p0 + kk] = -w[i];
             }
 #pragma unroll
         for (int i = jt; i < TILES; ++i)
@@ -195,6 +195,12 @@ __device__ __forceinline__ void eliminate_wave(d4 (&acc)[TILES * (TILES + 1) / 2
                   __builtin_amdgcn_mfma_f64_16x16x4f64(w[i], c[j], acc[i * (i + 1) / 2 + j], 0, 0, 0);
         wave_lds_fence(); // P is written again
       }
+}
+
+// Sum of the two doubles at the byte offsets in the halves of k.
+__device__ __forceinline__ double two(const double *pool, uint32_t k)
+{
+  return *(const double *)((const char *)pool + (k & 0xFFFF)) + *(const double *)((const char *)pool + (k >> 16));
 }
 
 // Lower tiles of a front of TILES tile rows dealt out to WR x WC waves, wave (wr, wc) holding
@@ -279,6 +285,37 @@ struct FrontTiles {
             }
   }
 
+  // Entry (r, c) of every tile = the sources that the tables name in the leaves' Schur complements.
+  __device__ __forceinline__ void assemble(const uint32_t *tables, const DirectFront &f, const double *pool, int tm, int lane)
+  {
+    const uint4 *tab = (const uint4 *)(tables + f.tab) + lane, *tabx = (const uint4 *)(tables + f.tabx) + lane;
+    uint4 s[A][B];
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+      for (int b = 0; b < B; ++b)
+        if (any(a, b))
+          {
+            const int i = min(WR * a + wr, tm - 1), j = min(WC * b + wc, i); // (a tile that is not there: another)
+            s[a][b] = tab[64 * (i * (i + 1) / 2 + j)];
+          }
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+      for (int b = 0; b < B; ++b)
+        if (any(a, b))
+          {
+            const uint4 &k = s[a][b];
+            acc[a][b] = (d4){two(pool, k.x), two(pool, k.y), two(pool, k.z), two(pool, k.w)};
+            const int q = (WR * a + wr) * (WR * a + wr + 1) / 2 + WC * b + wc;
+            if (mine(a, b, tm) && ((f.extra >> q) & 1))
+              {
+                const uint4 x = tabx[64 * __builtin_popcount(f.extra & ((1u << q) - 1))];
+                acc[a][b] += (d4){two(pool, x.x), two(pool, x.y), two(pool, x.z), two(pool, x.w)};
+              }
+          }
+  }
+
   // Entry (r, c) of every tile = sum over the children that have both rows; child(k, ra, ca, ok):
   // its entry, 0 if not ok.  code: byte k of row r = its row in child k, 255 = none.
   template <typename Child>
@@ -350,9 +387,11 @@ constexpr int kNp = 17; // nodes per side of a block
 // a block): its 9-node matrix with the centre of a full patch eliminated, and one right-hand
 // side, -sum_B S_Bc x(B) over the given values x (0 at the other nodes), plus the loads of the
 // nodes it owns.  All four waves form the matrix, each for its own right-hand side.
+// Then the pair's middle node: the partner patch is the neighbouring lane.
 struct Patch {
   double S[45], v[9], inv; // inv: 1 / the centre's diagonal, 0 without a centre
-  bool valid;
+  double s[9], invm;       // column of the pair's middle node; 1 / its diagonal, 0 without one
+  bool valid, full;
 
   // elem: the leaf's fine cells; x: block nodes from the patch's first one; load(lx, ly): the
   // load of a node of the leaf
@@ -382,7 +421,7 @@ struct Patch {
               S[tri(a, b)] -= c;
             }
         }
-    const bool full = 2 * px + 2 <= lf.w && 2 * py + 2 <= lf.h;
+    full = 2 * px + 2 <= lf.w && 2 * py + 2 <= lf.h;
     inv = full ? reciprocal(S[tri(4, 4)]) : 0.0;
 #pragma unroll
     for (int a = 0; a < 9; ++a)
@@ -420,55 +459,114 @@ struct Patch {
       }
   }
 
-  // to the leaf's pool: the matrix (by one wave), right-hand side i
+  static __device__ __forceinline__ double partner(double x) { return dpp_f64<0xB1>(x); } // quad_perm [1, 0, 3, 2]
+
+  // The middle node of the pair (node 5 of the left patch, 3 of the right one): its column, the
+  // right-hand side without it.
+  __device__ __forceinline__ void middle(const DirectLeaf &lf, int px, int py)
+  {
+    const bool odd = px & 1, merged = 2 * (px | 1) < lf.w && 2 * py + 2 <= lf.h;
+#pragma unroll
+    for (int b = 0; b < 9; ++b)
+      s[b] = b == 4 && full ? 0.0 : odd ? S[tri(b, 3)] : S[tri(b, 5)];
+    const double d = odd ? s[3] : s[5];
+    const double dm = d + partner(d);
+    // the two nodes that the patches share (2 and 8 of the left one, 0 and 6 of the right one)
+    // have both patches' part; what they alone take part in counts with the left patch
+    const double s0 = odd ? s[0] : s[2], s1 = odd ? s[6] : s[8], t0 = s0 + partner(s0), t1 = s1 + partner(s1);
+    s[0] = odd ? t0 : s[0];
+    s[2] = odd ? s[2] : t0;
+    s[6] = odd ? t1 : s[6];
+    s[8] = odd ? s[8] : t1;
+    invm = merged ? reciprocal(dm) : 0.0;
+    const double ve = odd ? v[3] : v[5];
+    const double q = (ve + partner(ve)) * invm;
+#pragma unroll
+    for (int b = 0; b < 9; ++b)
+      v[b] -= (b == 0 || b == 6) && odd ? 0.0 : s[b] * q;
+  }
+
+  // to the leaf's pool: the matrix without the middle node (by one wave), right-hand side i
   __device__ __forceinline__ void store(double *pool, int p, int i, bool matrix) const
   {
     double *o = pool + p * kPatchDoubles;
     if (matrix && p == 0)
       pool[kLeafDoubles - 1] = 0.0;
-    if (!valid)
+    if (valid)
+#pragma unroll
+      for (int c = 0; c < 9; ++c)
+        o[45 + i * 9 + c] = v[c];
+    if (!matrix)
       return;
-    if (matrix)
+    const bool odd = p & 1;
+    if (valid)
 #pragma unroll
-      for (int k = 0; k < 45; ++k)
-        o[k] = S[k];
+      for (int a = 0; a < 9; ++a)
+        {
+          const double t = s[a] * invm;
 #pragma unroll
-    for (int c = 0; c < 9; ++c)
-      o[45 + i * 9 + c] = v[c];
+          for (int b = 0; b <= a; ++b)
+            o[tri(a, b)] = S[tri(a, b)] - (a % 6 == 0 && b % 6 == 0 && odd ? 0.0 : t * s[b]);
+        }
+    // then the entries between the patches of the pair, in place of the eliminated nodes'
+    double l[5], r[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+      {
+        const double mine = kPairRight[k] == 5 && !full ? s[4] : s[kPairRight[k]], pr = partner(mine),
+                     pl = partner(s[kPairLeft[k]]);
+        l[k] = -(odd ? pl : s[kPairLeft[k]]) * invm;
+        r[k] = odd ? mine : pr;
+      }
+    if (invm != 0.0 && !odd)
+#pragma unroll
+      for (int e = 0; e < kPairSlotsLeft; ++e)
+        o[kPairSlot[e]] = l[e / 5] * r[e % 5];
+    if (invm != 0.0 && odd)
+#pragma unroll
+      for (int e = kPairSlotsLeft; e < 25; ++e)
+        o[kPairSlot[e]] = l[e / 5] * r[e % 5];
   }
 };
 
-// Tiles of a leaf's front from its patches.
+// Tiles of a leaf's front from its patches.  load() asks for the tables, without a branch around
+// any load, ahead of the work on the patches: waited for tile by tile they took 10k cycles.
 template <int TILES>
-__device__ __forceinline__ void leaf_front(const uint32_t *tables, const DirectLeafType &t, const double *pool, int m, int lane,
-                                           d4 (&acc)[TILES * (TILES + 1) / 2])
-{
-  const uint32_t *tab = tables + t.tab, *tabx = tables + t.tabx;
-  auto at = [&](uint32_t bytes) { return *(const double *)((const char *)pool + bytes); };
+struct LeafTables {
+  static constexpr int N = TILES * (TILES + 1) / 2;
+  uint4 s[N];
+
+  __device__ __forceinline__ void load(const uint32_t *tables, const DirectLeafType &t, int lane)
+  {
+    const uint4 *tab = (const uint4 *)(tables + t.tab) + lane;
 #pragma unroll
-  for (int i = 0, q = 0; i < TILES; ++i)
+    for (int q = 0; q < N; ++q)
+      s[q] = tab[64 * q];
+  }
+
+  __device__ __forceinline__ void front(const uint32_t *tables, const DirectLeafType &t, const double *pool, int lane,
+                                        d4 (&acc)[N]) const
+  {
+    const uint4 *tabx = (const uint4 *)(tables + t.tabx) + lane;
+    // entries of three or four patches are a patch corner's with itself and with the right-hand
+    // sides: in the first two tile columns
 #pragma unroll
-    for (int j = 0; j <= i; ++j, ++q)
-      {
-        acc[q] = (d4){0, 0, 0, 0};
-        if (16 * i < m)
-          {
+    for (int q = 0; q < N; ++q)
+      acc[q] = (d4){two(pool, s[q].x), two(pool, s[q].y), two(pool, s[q].z), two(pool, s[q].w)};
+    uint4 x[TILES][2];
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-              {
-                const uint32_t s = tab[(q * 4 + v) * 64 + lane];
-                acc[q][v] = at(s & 0xFFFF) + at(s >> 16);
-              }
-            if ((t.extra >> q) & 1)
+    for (int i = 0; i < TILES; ++i)
 #pragma unroll
-              for (int v = 0; v < 4; ++v)
-                {
-                  const uint32_t s = tabx[(q * 4 + v) * 64 + lane];
-                  acc[q][v] += at(s & 0xFFFF) + at(s >> 16);
-                }
-          }
-      }
-}
+      for (int j = 0; j <= i && j < 2; ++j)
+        x[i][j] = tabx[64 * (i * (i + 1) / 2 + j)];
+#pragma unroll
+    for (int i = 0; i < TILES; ++i)
+#pragma unroll
+      for (int j = 0; j <= i && j < 2; ++j)
+        if ((t.extra >> (i * (i + 1) / 2 + j)) & 1)
+          acc[i * (i + 1) / 2 + j] += (d4){two(pool, x[i][j].x), two(pool, x[i][j].y), two(pool, x[i][j].z), two(pool, x[i][j].w)};
+  }
+};
 
 // Node (t along side s) of a block's outline, s = bottom, top, left, right.
 __device__ __forceinline__ bool outline_node(const DirectFront &f, int s, int t, int &X, int &Y)
@@ -486,13 +584,12 @@ constexpr int kLeafWork = 16 * kLeafTiles * 4;  // pivot columns of a leaf
 // Bound by instruction issue (the 4 x 4 inverses and operand forming around the matrix
 // instructions), so what does not depend on the pivots is kept out of the pivot loops.
 template <int CELLS>
-__global__ void __launch_bounds__(kTpb, 2) direct_leaf_forward(DirectArgs a)
+__global__ void __launch_bounds__(kTpb, 3) direct_leaf_forward(DirectArgs a)
 {
   __shared__ double pool[4 * kLeafDoubles]; // fine cells; patches of the four leaves; their Schur complements
-  __shared__ double work[4 * kLeafWork];    // given values of the block's nodes; pivot columns
-  __shared__ uint32_t code[kBlockRows];
-  static_assert(6 * kElemCells <= 4 * kLeafDoubles && kDirectRhs * kNp * kNp <= 4 * kLeafWork &&
-                  2 * kBlockRows * 4 <= 4 * kLeafWork, "shared regions");
+  __shared__ double work[kDirectRhs * kNp * kNp]; // given values of the block's nodes; pivot columns
+  static_assert(6 * kElemCells <= 4 * kLeafDoubles && 4 * kLeafWork <= kDirectRhs * kNp * kNp &&
+                  2 * kBlockRows * 4 <= kDirectRhs * kNp * kNp && kLeafLd * kLeafLd < kLeafDoubles, "shared regions");
   const int nblk = a.n_fronts[a.depth - 1];
   const int slot = blockIdx.x / nblk;
   if (a.need && !a.need[slot])
@@ -503,8 +600,6 @@ __global__ void __launch_bounds__(kTpb, 2) direct_leaf_forward(DirectArgs a)
   const int m = f.ne + f.nb + kDirectRhs;
   const double *R = a.loads ? a.loads + (size_t)slot * kDirectRhs * np * np : nullptr;
   const bool touches = !R && (f.x0 == 0 || f.y0 == 0 || f.x0 + f.w == nf || f.y0 + f.h == nf);
-  for (int r = threadIdx.x; r < kBlockRows; r += kTpb)
-    code[r] = r < m ? a.tables[f.codes + r] : 0xFFFFFFFFu;
   if (touches)
     {
       for (int k = threadIdx.x; k < kDirectRhs * kNp * kNp; k += kTpb)
@@ -522,6 +617,8 @@ __global__ void __launch_bounds__(kTpb, 2) direct_leaf_forward(DirectArgs a)
         }
     }
   block_conductances<CELLS>(a, slot, cell, f, pool);
+  const DirectLeafType &t = a.types[a.leaves[f.child[wave]].fwd];
+  LeafTables<kLeafTiles> tab;
   __syncthreads();
   {
     const DirectLeaf &lf = a.leaves[f.child[lane >> 4]];
@@ -531,19 +628,20 @@ __global__ void __launch_bounds__(kTpb, 2) direct_leaf_forward(DirectArgs a)
     const int X = min(lf.x0 - f.x0 + 2 * px, kNp - 3), Y = min(lf.y0 - f.y0 + 2 * py, kNp - 3);
     p.form(lf, px, py, pool + elem_at(lane >> 4, 0, 0), touches, work + (wave * kNp + Y) * kNp + X, R != nullptr,
            [&](int lx, int ly) { return R[((size_t)wave * np + lf.y0 + ly) * np + lf.x0 + lx]; });
+    p.middle(lf, px, py);
     __syncthreads(); // fine cells and given values read by all
     p.store(pool + (lane >> 4) * kLeafDoubles, lane & 15, wave, wave == 0);
+    tab.load(a.tables, t, lane);
   }
   __syncthreads();
   {
-    const DirectLeafType &t = a.types[a.leaves[f.child[wave]].fwd];
     double *mine = pool + wave * kLeafDoubles;
     const int ne = t.ne, lm = ne + t.nb + kDirectRhs, l16 = lane & 15;
-    d4 acc[15];
-    leaf_front<kLeafTiles>(a.tables, t, mine, lm, lane, acc);
+    d4 acc[kLeafTiles * (kLeafTiles + 1) / 2];
+    tab.front(a.tables, t, mine, lane, acc);
     wave_lds_fence();
-    eliminate_wave<kLeafTiles, 36, false>(acc, ne, lm, work + wave * kLeafWork, nullptr, 0, lane);
-    // its Schur complement, whole, in place of its patches
+    eliminate_wave<kLeafTiles, kLeafElim, false>(acc, ne, lm, work + wave * kLeafWork, nullptr, lane);
+    // its Schur complement's lower part in place of its patches
 #pragma unroll
     for (int i = 0; i < kLeafTiles; ++i)
 #pragma unroll
@@ -554,10 +652,7 @@ __global__ void __launch_bounds__(kTpb, 2) direct_leaf_forward(DirectArgs a)
             {
               const int r = 16 * i + mfma_row(lane, v) - ne, c = 16 * j + l16 - ne;
               if (c >= 0 && (j < i || r >= c) && r < lm - ne)
-                {
-                  mine[r * kLeafLd + c] = acc[i * (i + 1) / 2 + j][v];
-                  mine[c * kLeafLd + r] = acc[i * (i + 1) / 2 + j][v];
-                }
+                mine[r * kLeafLd + c] = acc[i * (i + 1) / 2 + j][v];
             }
     if (lane == 0)
       mine[kLeafDoubles - 1] = 0.0; // what absent entries read
@@ -566,9 +661,7 @@ __global__ void __launch_bounds__(kTpb, 2) direct_leaf_forward(DirectArgs a)
   FrontTiles<kBlockTiles, 2, 2> front;
   front.wr = wave >> 1;
   front.wc = wave & 1;
-  front.assemble(code, f.kids, (m + 15) >> 4, lane, [&](int k, uint32_t ra, uint32_t ca, bool ok) {
-    return pool[k * kLeafDoubles + (ok ? ra * kLeafLd + ca : kLeafDoubles - 1)];
-  });
+  front.assemble(a.tables, f, pool, (m + 15) >> 4, lane);
   double *base = a.scratch + (size_t)slot * a.cell_doubles;
   front.eliminate(f.ne, m, work, base + f.w_off, f.ldw, lane);
   if (a.depth > 1)
@@ -618,14 +711,13 @@ __global__ void __launch_bounds__(64 * WR * WC, 2) direct_front(DirectArgs a)
 }
 
 // Rows ne-1..0 of the top-down pass of a front of at most MAXE <= 64 eliminated rows, lane p
-// holding row p: y = its four right-hand sides less the outline's part.  W: row r at W[r * ldw].
+// holding row p: y = its four right-hand sides less the outline's part, w[r] = W(r, p).
 template <int MAXE>
-__device__ __forceinline__ void back_rows(const double *W, int ldw, int ne, int lane, double (&y)[kDirectRhs])
+__device__ __forceinline__ void back_rows(double (&w)[MAXE], int ne, int lane, double (&y)[kDirectRhs])
 {
-  double w[MAXE];
 #pragma unroll
   for (int r = 0; r < MAXE; ++r)
-    w[r] = r < ne && (lane >> 2) < (r >> 2) ? W[(size_t)r * ldw + lane] : 0.0; // (a row's own pivot block: in W already)
+    w[r] = (lane >> 2) < (r >> 2) ? w[r] : 0.0; // (a row's own pivot block: in W already)
 #pragma unroll
   for (int r = MAXE - 1; r > 0; --r)
     if (r < ne)
@@ -723,14 +815,17 @@ __global__ void __launch_bounds__(64) direct_front_back(DirectArgs a)
 // centres.  The leaves are solved with their whole outline given: 33 rows instead of the 69 of
 // the bottom-up front, so forming them again costs less than storing 0.9 MB of W per 64^2 cell.
 template <int CELLS>
-__global__ void __launch_bounds__(kTpb, 2) direct_leaf_back(DirectArgs a)
+__global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
 {
-  constexpr int NP = kNp, LDW = 34, PW = 16 * kLeafBackTiles * 4;
+  constexpr int NP = kNp;
   __shared__ double X[kDirectRhs * NP * NP]; // the block's node values, 0 where not known yet
-  __shared__ double pool[4 * kLeafDoubles];  // fine cells; patches; each leaf's W
-  __shared__ double work[4 * PW + 64 * 9];   // the outline's part of the block's lines; pivot columns, patch centres
+  __shared__ double pool[4 * kLeafDoubles];  // fine cells, the outline's part of the block's lines; patches; each
+                                             // leaf's W and pivot columns
   __shared__ int at[kBlockRows];             // place in X of every row of the block's front
-  static_assert(8 * kDirectRhs * 32 <= 4 * PW + 64 * 9, "shared regions");
+  constexpr int kLeafW = (kLeafElim + kDirectRhs) * (kLeafElim + kDirectRhs + 1) / 2;
+  double *work = pool + 6 * kElemCells;
+  static_assert(6 * kElemCells + 8 * kDirectRhs * 32 <= 4 * kLeafDoubles &&
+                  kLeafW + 16 * kLeafBackTiles * 4 <= kLeafDoubles, "shared regions");
   const int nblk = a.n_fronts[a.depth - 1];
   const int slot = blockIdx.x / nblk;
   if (a.need && !a.need[slot])
@@ -741,28 +836,49 @@ __global__ void __launch_bounds__(kTpb, 2) direct_leaf_back(DirectArgs a)
   double *x = a.x_of(slot, cell);
   const double *R = a.loads ? a.loads + (size_t)slot * kDirectRhs * np * np : nullptr;
   const double *W = a.scratch + (size_t)slot * a.cell_doubles + f.w_off;
-  // the outline's part of the block's lines: thread (p, g) takes row p and outline rows g, g + 8, ...
-  const int p = threadIdx.x & 31, g = threadIdx.x >> 5;
-  double wo[8];
+  // Everything this launch reads is asked for here, without a branch around a load (places beyond
+  // a row or a side read a neighbour's and drop it): a load waited for where it is used costs
+  // ~1000 cycles, and the block's lines alone take 29 of them one after the other.
+  // The outline's part of the block's lines: thread (p, g) takes row p and outline rows g, g + 8, ...
+  const int p = threadIdx.x & 31, g = threadIdx.x >> 5, pw = min(p, f.ldw - 1);
+  double wo[8], wl[kBlockElim], wb[kDirectRhs], xo[2];
+  int xat[2];
 #pragma unroll
   for (int k = 0; k < 8; ++k)
-    wo[k] = p < f.ne && g + 8 * k < f.nb ? W[(size_t)(f.ne + g + 8 * k) * f.ldw + p] : 0.0;
+    wo[k] = W[(size_t)min(f.ne + g + 8 * k, f.ne + f.nb) * f.ldw + pw];
+  if (wave == 0)
+    {
+#pragma unroll
+      for (int r = 0; r < kBlockElim; ++r)
+        wl[r] = W[(size_t)min(r, f.ne) * f.ldw + pw];
+#pragma unroll
+      for (int i = 0; i < kDirectRhs; ++i)
+        wb[i] = W[(size_t)(f.ne + f.nb + i) * f.ldw + pw];
+    }
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    {
+      const int e = min((int)threadIdx.x + k * kTpb, kDirectRhs * 4 * NP - 1), i = e / (4 * NP);
+      int X0, Y0;
+      const bool ok = outline_node(f, e / NP & 3, e % NP, X0, Y0);
+      X0 = min(X0, f.w), Y0 = min(Y0, f.h);
+      xo[k] = x[((size_t)i * np + f.y0 + Y0) * np + f.x0 + X0];
+      xat[k] = ok ? (i * NP + Y0) * NP + X0 : -1;
+    }
+  const int node = a.tables[f.nodes + min((int)threadIdx.x, f.ne + f.nb - 1)];
+  const DirectLeafType &t = a.types[a.leaves[f.child[wave]].back];
+  LeafTables<kLeafBackTiles> tab;
+  tab.load(a.tables, t, lane);
   for (int k = threadIdx.x; k < kDirectRhs * NP * NP; k += kTpb)
     X[k] = 0;
-  if (threadIdx.x < f.ne + f.nb)
-    {
-      const int n = a.tables[f.nodes + threadIdx.x];
-      at[threadIdx.x] = (n / np - f.y0) * NP + n % np - f.x0;
-    }
   block_conductances<CELLS>(a, slot, cell, f, pool);
+  if (threadIdx.x < f.ne + f.nb)
+    at[threadIdx.x] = (node / np - f.y0) * NP + node % np - f.x0;
   __syncthreads();
-  for (int k = threadIdx.x; k < kDirectRhs * 4 * NP; k += kTpb)
-    {
-      const int i = k / (4 * NP);
-      int X0, Y0;
-      if (outline_node(f, k / NP & 3, k % NP, X0, Y0))
-        X[(i * NP + Y0) * NP + X0] = x[((size_t)i * np + f.y0 + Y0) * np + f.x0 + X0];
-    }
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    if (xat[k] >= 0)
+      X[xat[k]] = xo[k];
   __syncthreads();
   {
     double s[kDirectRhs] = {0, 0, 0, 0};
@@ -790,15 +906,16 @@ __global__ void __launch_bounds__(kTpb, 2) direct_leaf_back(DirectArgs a)
 #pragma unroll
           for (int k = 0; k < 8; ++k)
             s += work[(k * kDirectRhs + i) * 32 + (lane & 31)];
-          y[i] = lane < f.ne ? W[(size_t)(f.ne + f.nb + i) * f.ldw + lane] - s : 0.0;
+          y[i] = lane < f.ne ? wb[i] - s : 0.0;
         }
-      back_rows<kBlockElim>(W, f.ldw, f.ne, lane, y);
+      back_rows<kBlockElim>(wl, f.ne, lane, y);
       if (lane < f.ne)
 #pragma unroll
         for (int i = 0; i < kDirectRhs; ++i)
           X[i * NP * NP + at[lane]] = y[i];
     }
   __syncthreads();
+  double cc[9], cm[9], invm; // what the nodes eliminated in closed form need
   {
     const DirectLeaf &lf = a.leaves[f.child[lane >> 4]];
     const int px = lane & 3, py = (lane >> 2) & 3;
@@ -806,28 +923,35 @@ __global__ void __launch_bounds__(kTpb, 2) direct_leaf_back(DirectArgs a)
     Patch q;
     q.form(lf, px, py, pool + elem_at(lane >> 4, 0, 0), true, X + (wave * NP + Y0) * NP + X0, R != nullptr,
            [&](int lx, int ly) { return R[((size_t)wave * np + lf.y0 + ly) * np + lf.x0 + lx]; });
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+      cc[k] = k == 4 ? q.inv : q.S[tri(k, 4)];
+    q.middle(lf, px, py);
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+      cm[k] = k % 6 == 0 && (px & 1) ? 0.0 : q.s[k]; // (shared nodes: in the left patch's sum)
+    invm = q.invm;
     __syncthreads(); // fine cells read by all
     q.store(pool + (lane >> 4) * kLeafDoubles, lane & 15, wave, wave == 0);
-    if (wave == 0)
-#pragma unroll
-      for (int k = 0; k < 9; ++k)
-        work[4 * PW + lane * 9 + k] = k == 4 ? q.inv : q.S[tri(k, 4)];
   }
   __syncthreads();
   {
     const DirectLeaf &lf = a.leaves[f.child[wave]];
-    const DirectLeafType &t = a.types[lf.back];
     double *mine = pool + wave * kLeafDoubles;
     const int lm = t.ne + kDirectRhs;
-    d4 acc[6];
-    leaf_front<kLeafBackTiles>(a.tables, t, mine, lm, lane, acc);
+    d4 acc[kLeafBackTiles * (kLeafBackTiles + 1) / 2];
+    tab.front(a.tables, t, mine, lane, acc);
     wave_lds_fence();
-    eliminate_wave<kLeafBackTiles, 36, true>(acc, t.ne, lm, work + wave * PW, mine, LDW, lane);
+    eliminate_wave<kLeafBackTiles, kLeafElim, true>(acc, t.ne, lm, mine + kLeafW, mine, lane);
     double y[kDirectRhs];
 #pragma unroll
     for (int i = 0; i < kDirectRhs; ++i)
-      y[i] = lane < t.ne ? mine[(t.ne + i) * LDW + lane] : 0.0;
-    back_rows<33>(mine, LDW, t.ne, lane, y);
+      y[i] = lane < t.ne ? mine[(t.ne + i) * (t.ne + i + 1) / 2 + lane] : 0.0;
+    double w[kLeafElim];
+#pragma unroll
+    for (int r = 0; r < kLeafElim; ++r)
+      w[r] = mine[r * (r + 1) / 2 + min(lane, r)];
+    back_rows<kLeafElim>(w, t.ne, lane, y);
     if (lane < t.ne)
       {
         const uint32_t xy = a.tables[t.nodes + lane];
@@ -839,19 +963,32 @@ __global__ void __launch_bounds__(kTpb, 2) direct_leaf_back(DirectArgs a)
   }
   __syncthreads();
   {
-    // patch centres: thread = (patch, basis)
+    // middle nodes of the pairs, then patch centres: thread = (patch, basis)
     const DirectLeaf &lf = a.leaves[f.child[lane >> 4]];
     const int px = lane & 3, py = (lane >> 2) & 3;
-    if (2 * px + 2 <= lf.w && 2 * py + 2 <= lf.h)
+    const bool odd = px & 1, centre = 2 * px + 2 <= lf.w && 2 * py + 2 <= lf.h;
+    const int X0 = min(lf.x0 - f.x0 + 2 * px, NP - 3), Y0 = min(lf.y0 - f.y0 + 2 * py, NP - 3);
+    double *o = X + (wave * NP + Y0) * NP + X0;
+    const double *Rc = R ? R + ((size_t)wave * np + f.y0 + Y0 + 1) * np + f.x0 + X0 + 1 : nullptr; // the centre's load
+    const double rc = centre && R ? *Rc : 0.0;
+    double s = invm != 0.0 && R && !odd ? Rc[1] : 0.0; // the middle node's
+    if (centre)
+      s -= (odd ? cc[3] : cc[5]) * cc[4] * rc;
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+      s -= (k == (odd ? 3 : 5) ? 0.0 : cm[k]) * o[k / 3 * NP + k % 3];
+    s = (s + Patch::partner(s)) * invm;
+    if (invm != 0.0 && !odd)
+      o[NP + 2] = s;
+    wave_lds_fence();
+    if (centre)
       {
-        const double *c = work + 4 * PW + lane * 9;
-        double *o = X + (wave * NP + lf.y0 - f.y0 + 2 * py) * NP + lf.x0 - f.x0 + 2 * px;
-        double s = R ? R[((size_t)wave * np + lf.y0 + 2 * py + 1) * np + lf.x0 + 2 * px + 1] : 0.0;
+        s = rc;
 #pragma unroll
         for (int k = 0; k < 9; ++k)
           if (k != 4)
-            s -= c[k] * o[k / 3 * NP + k % 3];
-        o[NP + 1] = s * c[4];
+            s -= cc[k] * o[k / 3 * NP + k % 3];
+        o[NP + 1] = s * cc[4];
       }
   }
   __syncthreads();

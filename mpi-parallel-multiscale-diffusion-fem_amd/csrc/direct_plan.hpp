@@ -8,8 +8,9 @@
 // children, which it eliminates, then the nodes of its own outline that other
 // blocks share (Dirichlet nodes of the grid are never in a front), then the four
 // right-hand sides as four more rows.  A leaf is made of 2 x 2-cell patches whose
-// centre nodes are eliminated by closed formulas; its front holds its other
-// interior nodes and its outline.
+// centre nodes are eliminated by closed formulas, and so is the node in the middle
+// of the side that the two patches of a pair (side by side) share; its front holds
+// its other interior nodes and its outline.
 #pragma once
 
 #include <algorithm>
@@ -23,11 +24,22 @@ constexpr int kDirectMinNf = 9, kDirectMaxNf = 128; // resolutions with at least
 constexpr int kDirectRhs = 4;                      // bases of a 2D cell
 constexpr int kPatchDoubles = 81;                  // 3 x 3-node patch: 45 lower entries, then 4 x 9 right-hand sides
 constexpr int kLeafDoubles = 16 * kPatchDoubles + 1; // 16 patches and one zero (what table entries without a source read)
-constexpr int kLeafTiles = 5, kLeafBackTiles = 3;    // tile rows of a leaf's front: 33 + 32 + 4 and 33 + 4 rows
+constexpr int kLeafElim = 25;                        // most rows that a leaf's front eliminates
+constexpr int kLeafTiles = 4, kLeafBackTiles = 2;    // tile rows of a leaf's front: 25 + 32 + 4 and 25 + 4 rows
 constexpr int kLeafLd = 36;                          // leading dimension of a leaf's Schur complement (32 + 4)
 
 // Row of a 16 x 16 FP64 accumulator tile that entry v of lane l holds (its column is l % 16).
 constexpr int mfma_row(int lane, int v) { return (lane >> 4) + 4 * v; }
+
+// A pair's middle node (node 5 of the left patch, 3 of the right one) couples the nodes kPairLeft
+// of the left patch to the nodes kPairRight of the right one, neither of which the other has
+// (node 5, or node 4 where the right patch is one cell wide).  These 25 entries take the place of
+// the entries of the eliminated nodes: the first kPairSlotsLeft in the left patch, the others in
+// the right one.
+constexpr int kPairLeft[5] = {0, 1, 3, 6, 7}, kPairRight[5] = {1, 2, 5, 7, 8};
+constexpr int kPairSlotsLeft = 17;
+constexpr int kPairSlot[25] = {10, 11, 12, 13, 14, 19, 25, 32, 40, 15, 16, 17, 18, 20, 26, 33, 41, // (4, .), (5, .)
+                               6,  7,  8,  9,  18, 24, 31, 39};                                 // (3, .)
 
 struct DirectFront {
   int ne, nb;               // eliminated rows, outline rows (then kDirectRhs rows)
@@ -36,6 +48,9 @@ struct DirectFront {
   int codes;                // pool offset: byte k of row r = its row in child k's Schur complement, 255 = none
   int child[4];             // index of child k in the next level (leaf index on the last front level)
   int x0, y0, w, h;         // block, fine cells
+  int tab, tabx;            // (last front level) pool offsets: per (tile, lane, v) two 16-bit sources, bytes from
+                            // the four leaves' Schur complements; two more for the tiles in `extra`, in order
+  unsigned extra;
   uint8_t kids[20];         // bit k of tile row i: some of rows 16 i .. 16 i + 15 are in child k
   long long s_off, w_off;   // doubles from the cell's scratch
 };
@@ -47,7 +62,7 @@ struct DirectLeaf {
 struct DirectLeafType {
   int ne, nb;
   int nodes;                // pool offset: x | y << 8 (leaf coordinates) of every row < ne + nb
-  int tab, tabx;            // pool offsets: per (tile, v, lane) two 16-bit sources (bytes from the leaf's
+  int tab, tabx;            // pool offsets: per (tile, lane, v) two 16-bit sources (bytes from the leaf's
                             // patches); two more for the tiles in `extra`
   unsigned extra;
 };
@@ -189,6 +204,8 @@ public:
                 f.kids[r / 16] |= 1 << k;
           f.codes = (int)p.pool.size();
           p.pool.insert(p.pool.end(), code.begin(), code.end());
+          if (l + 1 == D)
+            block_tables(f, code);
         }
     return p;
   }
@@ -198,12 +215,59 @@ private:
   std::vector<int> cut; // leaf boundaries along an axis
   std::vector<std::vector<std::vector<int>>> parent_rows;
   std::map<int, int> type_of;
+  std::map<std::vector<uint32_t>, DirectFront> block_of;
 
   int at(int level, int i) const { return cut[i << (p.depth - level)]; }
   void block(int level, int bx, int by, int &x0, int &y0, int &w, int &h) const
   {
     x0 = at(level, bx), y0 = at(level, by);
     w = at(level, bx + 1) - x0, h = at(level, by + 1) - y0;
+  }
+  // Assembly tables of a last-level front; fronts with the same rows share them.
+  void block_tables(DirectFront &f, const std::vector<uint32_t> &code)
+  {
+    auto it = block_of.find(code);
+    if (it != block_of.end())
+      {
+        f.tab = it->second.tab, f.tabx = it->second.tabx, f.extra = it->second.extra;
+        return;
+      }
+    const int m = (int)code.size(), tiles = (m + 15) / 16;
+    std::vector<uint32_t> tab, tabx;
+    for (int i = 0, q = 0; i < tiles; ++i)
+      for (int j = 0; j <= i; ++j, ++q)
+        {
+          std::vector<uint32_t> more;
+          bool any = false;
+          for (int lane = 0; lane < 64; ++lane)
+            for (int v = 0; v < 4; ++v)
+              {
+                uint32_t s[4];
+                s[0] = s[1] = s[2] = s[3] = 4 * kLeafDoubles - 1;
+                const int r = 16 * i + mfma_row(lane, v), c = 16 * j + lane % 16;
+                if (r < m && c < m)
+                  for (int k = 0, n = 0; k < 4; ++k)
+                    {
+                      const uint32_t a = (code[r] >> (8 * k)) & 255, b = (code[c] >> (8 * k)) & 255;
+                      if (a != 255 && b != 255)
+                        s[n++] = k * kLeafDoubles + std::max(a, b) * kLeafLd + std::min(a, b);
+                    }
+                tab.push_back(8 * s[0] | 8 * s[1] << 16);
+                more.push_back(8 * s[2] | 8 * s[3] << 16);
+                any = any || s[2] != 4 * kLeafDoubles - 1;
+              }
+          if (any)
+            {
+              f.extra |= 1u << q;
+              tabx.insert(tabx.end(), more.begin(), more.end());
+            }
+        }
+    p.pool.resize((p.pool.size() + 3) & ~(size_t)3); // (read four at a time)
+    f.tab = (int)p.pool.size();
+    p.pool.insert(p.pool.end(), tab.begin(), tab.end());
+    f.tabx = (int)p.pool.size();
+    p.pool.insert(p.pool.end(), tabx.begin(), tabx.end());
+    block_of[code] = f;
   }
   bool on_outline(int x0, int y0, int w, int h, int x, int y) const
   {
@@ -228,7 +292,8 @@ private:
               const bool given = (x == 0 && (sides & 1)) || (x == w && (sides & 2)) || (y == 0 && (sides & 4)) ||
                                  (y == h && (sides & 8));
               const bool centre = (x & 1) && (y & 1) && !edge; // of a full patch: an odd node inside is followed by a cell
-              if (given || (pass == 0 ? edge || centre : !edge))
+              const bool middle = x % 4 == 2 && (y & 1) && !edge; // of a pair, likewise
+              if (given || (pass == 0 ? edge || centre || middle : !edge))
                 continue;
               row_x.push_back(x), row_y.push_back(y);
             }
@@ -264,12 +329,32 @@ private:
             const int a = rx + 3 * ry, hi = std::max(a, b), lo = std::min(a, b);
             s[k++] = base + hi * (hi + 1) / 2 + lo;
           }
+      if (r < n) // coupled through a pair's middle node
+        for (int py = 0; py < ph; ++py)
+          for (int px = 0; px + 1 < pw; px += 2)
+            {
+              if (2 * py + 2 > h)
+                continue;
+              const int left = row_x[r] < row_x[c] ? r : c, right = r + c - left;
+              const int lx = row_x[left] - 2 * px, ly = row_y[left] - 2 * py;
+              const int rx = row_x[right] - 2 * px - 2, ry = row_y[right] - 2 * py;
+              if (lx < 0 || lx > 1 || rx < 1 || rx > 2 || ly < 0 || ly > 2 || ry < 0 || ry > 2)
+                continue;
+              int li = 0, ri = 0;
+              while (kPairLeft[li] != lx + 3 * ly)
+                ++li;
+              const int rn = rx + 3 * ry;
+              while (kPairRight[ri] != (rn == 4 ? 5 : rn))
+                ++ri;
+              const int e = li * 5 + ri;
+              s[k++] = (py * 4 + px + (e < kPairSlotsLeft ? 0 : 1)) * kPatchDoubles + kPairSlot[e];
+            }
     };
     std::vector<uint32_t> tab, tabx;
     for (int i = 0, q = 0; i < tiles; ++i)
       for (int j = 0; j <= i; ++j, ++q)
-        for (int v = 0; v < 4; ++v)
-          for (int lane = 0; lane < 64; ++lane)
+        for (int lane = 0; lane < 64; ++lane)
+          for (int v = 0; v < 4; ++v)
             {
               uint32_t s[4];
               sources(16 * i + mfma_row(lane, v), 16 * j + lane % 16, s);
@@ -278,6 +363,7 @@ private:
               if (s[2] != none)
                 t.extra |= 1u << q;
             }
+    p.pool.resize((p.pool.size() + 3) & ~(size_t)3); // (read four at a time)
     t.tab = (int)p.pool.size();
     p.pool.insert(p.pool.end(), tab.begin(), tab.end());
     t.tabx = (int)p.pool.size();
