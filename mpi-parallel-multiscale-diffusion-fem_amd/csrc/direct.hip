@@ -361,10 +361,10 @@ struct FrontTiles {
 
 // ---- leaves -------------------------------------------------------------------------------
 
-// Place of fine cell (lx, ly) of leaf q in an array of fine cells: the padding spreads the
-// patches' reads (every second cell of every second row) over the LDS banks.
-constexpr int kElemCells = 4 * 73;
-__device__ __forceinline__ constexpr int elem_at(int q, int lx, int ly) { return q * 73 + ly * 9 + lx; }
+// Place of fine cell (lx, ly) of leaf q in an array of fine cells: the padding puts the 32
+// patches' reads (every second cell of every second row) on 32 different pairs of LDS banks.
+constexpr int kElemRow = 12, kElemLeaf = 97, kElemCells = 4 * kElemLeaf;
+__device__ __forceinline__ constexpr int elem_at(int q, int lx, int ly) { return q * kElemLeaf + ly * kElemRow + lx; }
 
 // Fine-cell conductances of a <= 16 x 16 block into elem[6][kElemCells] (leaf q: children
 // (q & 1, q >> 1)), thread per fine cell; zero beyond a leaf.
@@ -381,7 +381,7 @@ __device__ __forceinline__ void block_conductances(const DirectArgs &a, int slot
     elem[k * kElemCells + elem_at(q, lx, ly)] = c[k];
 }
 
-constexpr int kNp = 17; // nodes per side of a block
+constexpr int kNp = 17, kNx = 20; // nodes per side of a block; row of its nodes' values (padded like the fine cells)
 
 // One 2 x 2 patch of a leaf (lane: leaf lane >> 4, patch lane & 15: a wave has the 64 patches of
 // a block): its 9-node matrix with the centre of a full patch eliminated, and one right-hand
@@ -439,7 +439,7 @@ struct Patch {
 #pragma unroll
       for (int b = 0; b < 9; ++b)
         {
-          const double xb = x[b / 3 * kNp + b % 3];
+          const double xb = x[b / 3 * kNx + b % 3];
 #pragma unroll
           for (int c = 0; c < 9; ++c)
             v[c] -= S[tri(b, c)] * xb;
@@ -576,6 +576,7 @@ __device__ __forceinline__ bool outline_node(const DirectFront &f, int s, int t,
   return X <= f.w && Y <= f.h;
 }
 
+constexpr int kLdsThird = 42 * 1280; // most LDS of a workgroup of which a CU holds three (160 KB in units of 1280 B)
 constexpr int kBlockTiles = 7, kBlockElim = 29; // a 16 x 16 block's front: 29 + 64 + 4 rows
 constexpr int kBlockRows = 16 * 8;              // (in tiles dealt out to 2 x 2 waves)
 constexpr int kLeafWork = 16 * kLeafTiles * 4;  // pivot columns of a leaf
@@ -587,9 +588,10 @@ template <int CELLS>
 __global__ void __launch_bounds__(kTpb, 3) direct_leaf_forward(DirectArgs a)
 {
   __shared__ double pool[4 * kLeafDoubles]; // fine cells; patches of the four leaves; their Schur complements
-  __shared__ double work[kDirectRhs * kNp * kNp]; // given values of the block's nodes; pivot columns
-  static_assert(6 * kElemCells <= 4 * kLeafDoubles && 4 * kLeafWork <= kDirectRhs * kNp * kNp &&
-                  2 * kBlockRows * 4 <= kDirectRhs * kNp * kNp && kLeafLd * kLeafLd < kLeafDoubles, "shared regions");
+  __shared__ double work[kDirectRhs * kNp * kNx]; // given values of the block's nodes; pivot columns
+  static_assert(6 * kElemCells <= 4 * kLeafDoubles && 4 * kLeafWork <= kDirectRhs * kNp * kNx &&
+                  2 * kBlockRows * 4 <= kDirectRhs * kNp * kNx && kLeafLd * kLeafLd < kLeafDoubles &&
+                  sizeof(pool) + sizeof(work) <= kLdsThird, "shared regions");
   const int nblk = a.n_fronts[a.depth - 1];
   const int slot = blockIdx.x / nblk;
   if (a.need && !a.need[slot])
@@ -602,7 +604,7 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_forward(DirectArgs a)
   const bool touches = !R && (f.x0 == 0 || f.y0 == 0 || f.x0 + f.w == nf || f.y0 + f.h == nf);
   if (touches)
     {
-      for (int k = threadIdx.x; k < kDirectRhs * kNp * kNp; k += kTpb)
+      for (int k = threadIdx.x; k < kDirectRhs * kNp * kNx; k += kTpb)
         work[k] = 0;
       __syncthreads();
       // the Dirichlet values on the block's outline
@@ -613,7 +615,7 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_forward(DirectArgs a)
           int X, Y;
           if (outline_node(f, k / kNp & 3, k % kNp, X, Y) &&
               (f.x0 + X == 0 || f.y0 + Y == 0 || f.x0 + X == nf || f.y0 + Y == nf))
-            work[(i * kNp + Y) * kNp + X] = x[((size_t)i * np + f.y0 + Y) * np + f.x0 + X];
+            work[(i * kNp + Y) * kNx + X] = x[((size_t)i * np + f.y0 + Y) * np + f.x0 + X];
         }
     }
   block_conductances<CELLS>(a, slot, cell, f, pool);
@@ -626,7 +628,7 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_forward(DirectArgs a)
     Patch p;
     // (a patch beyond its leaf reads within work and pool and is not stored)
     const int X = min(lf.x0 - f.x0 + 2 * px, kNp - 3), Y = min(lf.y0 - f.y0 + 2 * py, kNp - 3);
-    p.form(lf, px, py, pool + elem_at(lane >> 4, 0, 0), touches, work + (wave * kNp + Y) * kNp + X, R != nullptr,
+    p.form(lf, px, py, pool + elem_at(lane >> 4, 0, 0), touches, work + (wave * kNp + Y) * kNx + X, R != nullptr,
            [&](int lx, int ly) { return R[((size_t)wave * np + lf.y0 + ly) * np + lf.x0 + lx]; });
     p.middle(lf, px, py);
     __syncthreads(); // fine cells and given values read by all
@@ -817,15 +819,16 @@ __global__ void __launch_bounds__(64) direct_front_back(DirectArgs a)
 template <int CELLS>
 __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
 {
-  constexpr int NP = kNp;
-  __shared__ double X[kDirectRhs * NP * NP]; // the block's node values, 0 where not known yet
+  constexpr int NP = kNp, NX = kNx;
+  __shared__ double X[kDirectRhs * NP * NX]; // the block's node values, 0 where not known yet
   __shared__ double pool[4 * kLeafDoubles];  // fine cells, the outline's part of the block's lines; patches; each
                                              // leaf's W and pivot columns
-  __shared__ int at[kBlockRows];             // place in X of every row of the block's front
+  __shared__ int at[96];                     // place in X of every row (<= 93) of the block's front
   constexpr int kLeafW = (kLeafElim + kDirectRhs) * (kLeafElim + kDirectRhs + 1) / 2;
   double *work = pool + 6 * kElemCells;
   static_assert(6 * kElemCells + 8 * kDirectRhs * 32 <= 4 * kLeafDoubles &&
-                  kLeafW + 16 * kLeafBackTiles * 4 <= kLeafDoubles, "shared regions");
+                  kLeafW + 16 * kLeafBackTiles * 4 <= kLeafDoubles &&
+                  sizeof(X) + sizeof(pool) + sizeof(at) <= kLdsThird, "shared regions");
   const int nblk = a.n_fronts[a.depth - 1];
   const int slot = blockIdx.x / nblk;
   if (a.need && !a.need[slot])
@@ -863,17 +866,17 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
       const bool ok = outline_node(f, e / NP & 3, e % NP, X0, Y0);
       X0 = min(X0, f.w), Y0 = min(Y0, f.h);
       xo[k] = x[((size_t)i * np + f.y0 + Y0) * np + f.x0 + X0];
-      xat[k] = ok ? (i * NP + Y0) * NP + X0 : -1;
+      xat[k] = ok ? (i * NP + Y0) * NX + X0 : -1;
     }
   const int node = a.tables[f.nodes + min((int)threadIdx.x, f.ne + f.nb - 1)];
   const DirectLeafType &t = a.types[a.leaves[f.child[wave]].back];
   LeafTables<kLeafBackTiles> tab;
   tab.load(a.tables, t, lane);
-  for (int k = threadIdx.x; k < kDirectRhs * NP * NP; k += kTpb)
+  for (int k = threadIdx.x; k < kDirectRhs * NP * NX; k += kTpb)
     X[k] = 0;
   block_conductances<CELLS>(a, slot, cell, f, pool);
   if (threadIdx.x < f.ne + f.nb)
-    at[threadIdx.x] = (node / np - f.y0) * NP + node % np - f.x0;
+    at[threadIdx.x] = (node / np - f.y0) * NX + node % np - f.x0;
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < 2; ++k)
@@ -889,7 +892,7 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
           const int o = at[f.ne + g + 8 * k];
 #pragma unroll
           for (int i = 0; i < kDirectRhs; ++i)
-            s[i] += wo[k] * X[i * NP * NP + o];
+            s[i] += wo[k] * X[i * NP * NX + o];
         }
 #pragma unroll
     for (int i = 0; i < kDirectRhs; ++i)
@@ -912,7 +915,7 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
       if (lane < f.ne)
 #pragma unroll
         for (int i = 0; i < kDirectRhs; ++i)
-          X[i * NP * NP + at[lane]] = y[i];
+          X[i * NP * NX + at[lane]] = y[i];
     }
   __syncthreads();
   double cc[9], cm[9], invm; // what the nodes eliminated in closed form need
@@ -921,7 +924,7 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
     const int px = lane & 3, py = (lane >> 2) & 3;
     const int X0 = min(lf.x0 - f.x0 + 2 * px, NP - 3), Y0 = min(lf.y0 - f.y0 + 2 * py, NP - 3);
     Patch q;
-    q.form(lf, px, py, pool + elem_at(lane >> 4, 0, 0), true, X + (wave * NP + Y0) * NP + X0, R != nullptr,
+    q.form(lf, px, py, pool + elem_at(lane >> 4, 0, 0), true, X + (wave * NP + Y0) * NX + X0, R != nullptr,
            [&](int lx, int ly) { return R[((size_t)wave * np + lf.y0 + ly) * np + lf.x0 + lx]; });
 #pragma unroll
     for (int k = 0; k < 9; ++k)
@@ -955,10 +958,10 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
     if (lane < t.ne)
       {
         const uint32_t xy = a.tables[t.nodes + lane];
-        const int o = (lf.y0 - f.y0 + (int)(xy >> 8)) * NP + lf.x0 - f.x0 + (int)(xy & 255);
+        const int o = (lf.y0 - f.y0 + (int)(xy >> 8)) * NX + lf.x0 - f.x0 + (int)(xy & 255);
 #pragma unroll
         for (int i = 0; i < kDirectRhs; ++i)
-          X[i * NP * NP + o] = y[i];
+          X[i * NP * NX + o] = y[i];
       }
   }
   __syncthreads();
@@ -968,7 +971,7 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
     const int px = lane & 3, py = (lane >> 2) & 3;
     const bool odd = px & 1, centre = 2 * px + 2 <= lf.w && 2 * py + 2 <= lf.h;
     const int X0 = min(lf.x0 - f.x0 + 2 * px, NP - 3), Y0 = min(lf.y0 - f.y0 + 2 * py, NP - 3);
-    double *o = X + (wave * NP + Y0) * NP + X0;
+    double *o = X + (wave * NP + Y0) * NX + X0;
     const double *Rc = R ? R + ((size_t)wave * np + f.y0 + Y0 + 1) * np + f.x0 + X0 + 1 : nullptr; // the centre's load
     const double rc = centre && R ? *Rc : 0.0;
     double s = invm != 0.0 && R && !odd ? Rc[1] : 0.0; // the middle node's
@@ -976,10 +979,10 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
       s -= (odd ? cc[3] : cc[5]) * cc[4] * rc;
 #pragma unroll
     for (int k = 0; k < 9; ++k)
-      s -= (k == (odd ? 3 : 5) ? 0.0 : cm[k]) * o[k / 3 * NP + k % 3];
+      s -= (k == (odd ? 3 : 5) ? 0.0 : cm[k]) * o[k / 3 * NX + k % 3];
     s = (s + Patch::partner(s)) * invm;
     if (invm != 0.0 && !odd)
-      o[NP + 2] = s;
+      o[NX + 2] = s;
     wave_lds_fence();
     if (centre)
       {
@@ -987,8 +990,8 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
 #pragma unroll
         for (int k = 0; k < 9; ++k)
           if (k != 4)
-            s -= cc[k] * o[k / 3 * NP + k % 3];
-        o[NP + 1] = s * cc[4];
+            s -= cc[k] * o[k / 3 * NX + k % 3];
+        o[NX + 1] = s * cc[4];
       }
   }
   __syncthreads();
@@ -996,7 +999,7 @@ __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
     {
       const int i = k >> 8, X0 = k & 15, Y0 = (k >> 4) & 15;
       if (X0 > 0 && Y0 > 0 && X0 < f.w && Y0 < f.h)
-        x[((size_t)i * np + f.y0 + Y0) * np + f.x0 + X0] = X[(i * NP + Y0) * NP + X0];
+        x[((size_t)i * np + f.y0 + Y0) * np + f.x0 + X0] = X[(i * NP + Y0) * NX + X0];
     }
 }
 

@@ -23,7 +23,9 @@ namespace msfem {
 constexpr int kDirectMinNf = 9, kDirectMaxNf = 128; // resolutions with at least one cut and at most 17 tile rows
 constexpr int kDirectRhs = 4;                      // bases of a 2D cell
 constexpr int kPatchDoubles = 81;                  // 3 x 3-node patch: 45 lower entries, then 4 x 9 right-hand sides
-constexpr int kLeafDoubles = 16 * kPatchDoubles + 1; // 16 patches and one zero (what table entries without a source read)
+constexpr int kLeafDoubles = 1328; // 16 patches and a last zero (what table entries without a source read), padded so
+                                   // that two leaves' patches are in different LDS banks (1328 = 16 mod 32)
+static_assert(16 * kPatchDoubles < kLeafDoubles);
 constexpr int kLeafElim = 25;                        // most rows that a leaf's front eliminates
 constexpr int kLeafTiles = 4, kLeafBackTiles = 2;    // tile rows of a leaf's front: 25 + 32 + 4 and 25 + 4 rows
 constexpr int kLeafLd = 36;                          // leading dimension of a leaf's Schur complement (32 + 4)
