@@ -317,43 +317,58 @@ struct FrontTiles {
   }
 
   // Entry (r, c) of every tile = sum over the children that have both rows; child(k, ra, ca, ok):
-  // its entry, 0 if not ok.  code: byte k of row r = its row in child k, 255 = none.
+  // its entry, 0 if not ok.  code: byte k of row r = its row in child k, 255 = none.  A tile
+  // column's loads from a child are all on their way before the first is used (128-row fronts:
+  // 352 -> 314 us for 4076 with this and without a branch around each load).
   template <typename Child>
   __device__ __forceinline__ void assemble(const uint32_t *code, const uint8_t *kids, int tm, int lane, Child child)
   {
+    uint32_t rc[A][4];
+    int ka[A];
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+      {
+        ka[a] = WR * a + wr < tm ? kids[WR * a + wr] : 0;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          rc[a][v] = code[16 * (WR * a + wr) + mfma_row(lane, v)];
+      }
 #pragma unroll
     for (int b = 0; b < B; ++b)
       {
-        const uint32_t cc = WC * b + wc < tm ? code[16 * (WC * b + wc) + (lane & 15)] : 0xFFFFFFFFu;
+        const int kb = WC * b + wc < tm ? kids[WC * b + wc] : 0;
+        const uint32_t cc = code[16 * (WC * b + wc) + (lane & 15)];
 #pragma unroll
         for (int a = 0; a < A; ++a)
           if (any(a, b))
+            acc[a][b] = (d4){0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if ((kb >> k) & 1)
             {
-              acc[a][b] = (d4){0, 0, 0, 0};
-              if (mine(a, b, tm))
-                {
-                  uint32_t rc[4];
+              const uint32_t ca = (cc >> (8 * k)) & 255;
+              double t[A][4];
+#pragma unroll
+              for (int a = 0; a < A; ++a)
+                if (any(a, b))
+                  {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                      t[a][v] = 0;
+                    if (mine(a, b, tm) && ((ka[a] >> k) & 1))
+#pragma unroll
+                      for (int v = 0; v < 4; ++v)
+                        {
+                          const uint32_t ra = (rc[a][v] >> (8 * k)) & 255;
+                          t[a][v] = child(k, ra, ca, ra != kNone && ca != kNone);
+                        }
+                  }
+#pragma unroll
+              for (int a = 0; a < A; ++a)
+                if (any(a, b))
 #pragma unroll
                   for (int v = 0; v < 4; ++v)
-                    rc[v] = code[16 * (WR * a + wr) + mfma_row(lane, v)];
-                  const int both = kids[WR * a + wr] & kids[WC * b + wc];
-#pragma unroll
-                  for (int k = 0; k < 4; ++k)
-                    if ((both >> k) & 1)
-                      {
-                        const uint32_t ca = (cc >> (8 * k)) & 255;
-                        double t[4]; // all four on their way before the first is used
-#pragma unroll
-                        for (int v = 0; v < 4; ++v)
-                          {
-                            const uint32_t ra = (rc[v] >> (8 * k)) & 255;
-                            t[v] = child(k, ra, ca, ra != kNone && ca != kNone);
-                          }
-#pragma unroll
-                        for (int v = 0; v < 4; ++v)
-                          acc[a][b][v] += t[v];
-                      }
-                }
+                    acc[a][b][v] += t[a][v];
             }
       }
   }
@@ -582,8 +597,11 @@ constexpr int kBlockRows = 16 * 8;              // (in tiles dealt out to 2 x 2 
 constexpr int kLeafWork = 16 * kLeafTiles * 4;  // pivot columns of a leaf
 
 // Bottom-up pass of one block of the last front level: its four leaves, then its own front.
-// Bound by instruction issue (the 4 x 4 inverses and operand forming around the matrix
-// instructions), so what does not depend on the pivots is kept out of the pivot loops.
+// Bound by latency and issue together: of the 31k cycles of a CU that a block takes, the LDS is
+// busy for 15k, each SIMD's vector pipe for 11k and its matrix pipe for 5k.  Three workgroups a CU,
+// which 10 tiles a leaf and 53 KB of LDS admit, cover each other's waits; what does not depend on
+// the pivots is kept out of the pivot loops.  16304 blocks of 64^2 cells: 876 us, against 1250 with
+// two workgroups a CU, leaf fronts of 69 rows and row codes in place of the tables.
 template <int CELLS>
 __global__ void __launch_bounds__(kTpb, 3) direct_leaf_forward(DirectArgs a)
 {
@@ -702,10 +720,10 @@ __global__ void __launch_bounds__(64 * WR * WC, 2) direct_front(DirectArgs a)
   front.wr = wave / WC;
   front.wc = wave % WC;
   front.assemble(code, f.kids, (m + 15) >> 4, lane, [&](int k, uint32_t ra, uint32_t ca, bool ok) {
-    double v = 0;
-    if (ok) // a child keeps the rows in this order: its lower part
-      v = S[k][(ra > ca ? ra : ca) * ld[k] + (ra > ca ? ca : ra)];
-    return v;
+    // a child keeps the rows in this order: its lower part.  (No branch around the load, which
+    // would be waited for before the next.)
+    const double v = S[k][ok ? max(ra, ca) * ld[k] + min(ra, ca) : 0];
+    return ok ? v : 0.0;
   });
   front.eliminate(f.ne, m, P, base + f.w_off, f.ldw, lane);
   if (a.level > 0)
@@ -814,8 +832,10 @@ __global__ void __launch_bounds__(64) direct_front_back(DirectArgs a)
 }
 
 // Top-down pass of one block of the last front level: its own lines, its leaves, the patch
-// centres.  The leaves are solved with their whole outline given: 33 rows instead of the 69 of
-// the bottom-up front, so forming them again costs less than storing 0.9 MB of W per 64^2 cell.
+// centres.  The leaves are solved with their whole outline given: 29 rows instead of the 61 of
+// the bottom-up front, so forming them again costs less than storing their W.  Bound by the LDS
+// (10k of the 17k cycles a block); 16304 blocks: 432 us, against 812 with two workgroups a CU, each
+// of the block's rows loaded behind a branch and 2 x 2 patches alone eliminated in closed form.
 template <int CELLS>
 __global__ void __launch_bounds__(kTpb, 3) direct_leaf_back(DirectArgs a)
 {
@@ -1348,11 +1368,14 @@ static size_t direct_cell_doubles(const DirectHost &h, bool stored)
 // Whether a class reads stored fine cells (see kStored).
 static bool direct_stored(int coef_kind, bool general) { return general || coef_kind > 1; }
 
-// Cells solved together: as many as keep their scratch within ~1.5 GB, so that a batch of any
-// size needs no more.
+// Cells solved together: as many as keep their scratch within 4.5 GB of the 288, so that a batch of
+// any size needs no more.  A chunk is ~20 launches, whose upper levels have 1, 4, 16 fronts a cell
+// and end in partly empty waves of workgroups, so fewer are better: 4096 cells of 64^2 take 13.5 ms
+// with 0.25 GB, 9.28 with 1.5, 8.81 with 4.5 and 8.61 with 6.4.
+constexpr size_t kChunkDoubles = 560000000;
 static int direct_chunk(const DirectHost &h, int n_cells, bool stored)
 {
-  return (int)std::min<size_t>(n_cells, std::max<size_t>(16, 190000000 / direct_cell_doubles(h, stored)));
+  return (int)std::min<size_t>(n_cells, std::max<size_t>(16, kChunkDoubles / direct_cell_doubles(h, stored)));
 }
 
 size_t direct_scratch_doubles(const DirectHost &h, int n_cells, int coef_kind, bool general)
