@@ -264,6 +264,12 @@ hipError_t launch_coarse_assemble(int dim, int nc, const double *Ae, const doubl
 // systems of 2..128 cells per side reach 1e-13 in at most 10.
 constexpr int kMgIterations = 16;
 
+// Up to this many cells per side the Jacobi CG of one workgroup is done before the multigrid's
+// chain of launches, in 2D and 3D (us, multigrid / Jacobi, zero and reference boundary data): 3D 3
+// 228, 328 / 57, 120; 7 799, 829 / 211, 330; 11 1184, 1255 / 703, 1137; 12 1184, 1253 / 887, 1688;
+// 2D 5 139, 160 / 77, 99; 11 232, 236 / 168, 220; 12 229, 235 / 191, 246.
+constexpr int kJacobiMaxCells = 11;
+
 static size_t jacobi_work_doubles(int dim, int nc)
 {
   const size_t np = nc + 1;
@@ -279,7 +285,10 @@ static bool halves_evenly(int dim, int nc)
   return (dim == 2 ? (nc + 1) * (nc + 1) : (nc + 1) * (nc + 1) * (nc + 1)) <= 343;
 }
 
-size_t coarse_solve_work_doubles(int dim, int nc) { return (size_t)mg_layout(dim, nc).total; }
+size_t coarse_solve_work_doubles(int dim, int nc)
+{
+  return std::max((size_t)mg_layout(dim, nc).total, jacobi_work_doubles(dim, nc));
+}
 
 size_t coarse_solve_least_doubles(int dim, int nc)
 {
@@ -295,11 +304,12 @@ static hipError_t coarse_solve(int nc, const double *Kc, const double *Fc, const
   const MgLayout g = mg_layout(DIM, nc);
   CgVectors v;
   const MgState *state = nullptr;
-  if ((size_t)g.total <= work_doubles)
+  if (nc > kJacobiMaxCells && (size_t)g.total <= work_doubles)
     {
       hipError_t e = launch_mg_setup(DIM, g, Kc, Fc, cmask, cval, rel_tol, max_iter, work, st);
-      if (e == hipSuccess && g.tail == 0)
-        return launch_mg_small(DIM, g, Kc, u, iters, work, st);
+      if constexpr (DIM == 2) // (3D grids beyond kJacobiMaxCells do not fit one workgroup)
+        if (e == hipSuccess && g.tail == 0)
+          return launch_mg_small(g, Kc, u, iters, work, st);
       if (e == hipSuccess)
         e = launch_mg_iterations(DIM, g, kMgIterations, Kc, work, st);
       if (e != hipSuccess)

@@ -447,8 +447,8 @@ int class_variant(msfem_ctx *ctx, const msfem_batch *in, const msfem_solver_opts
 
 // Whether size class k runs the direct solves: box cells and quadrilaterals of 9..128 fine cells
 // per side at the default options.  A caller's x0, an explicit launch shape or another
-// coarse_space asks for the iterative solve.  64^2 cells in FP32 keep it too (4096 cells: 5.0 ms
-// against 8.9 ms direct), and so do classes of fewer than 32 cells of 64^2: those are what
+// coarse_space asks for the iterative solve.  64^2 cells in FP32 keep it too (4096 cells of a
+// Gaussian field: 5.1 ms against about 8 direct), and so do classes of fewer than 32 cells of 64^2: those are what
 // callers compare starts, preconditioners and iteration counts on.
 constexpr int kDirect64Cells = 32;
 bool class_direct(const Plan &p, const msfem_batch *in, const msfem_solver_opts *o, size_t k)
@@ -1630,7 +1630,7 @@ int msfem_fine_solve(msfem_ctx *ctx, int dim, int n, int coef_kind, const double
   hipError_t e = hipSuccess;
   if (g.tail == 0)
     {
-      HIP_TRY(ctx, launch_mg_small(2, g, Kc, du, dit, w, st));
+      HIP_TRY(ctx, launch_mg_small(g, Kc, du, dit, w, st));
       x = du;
       e = hipMemcpyAsync(&host, w + g.off_state, sizeof host, hipMemcpyDeviceToHost, st);
       if (e == hipSuccess)

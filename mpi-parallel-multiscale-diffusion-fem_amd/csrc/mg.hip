@@ -977,12 +977,9 @@ hipError_t launch_mg_iterations(int dim, const MgLayout &g, int count, const dou
   return dim == 2 ? iterations<2>(g, count, Kc, w, st) : iterations<3>(g, count, Kc, w, st);
 }
 
-hipError_t launch_mg_small(int dim, const MgLayout &g, const double *Kc, double *u, int *iters, double *w, hipStream_t st)
+hipError_t launch_mg_small(const MgLayout &g, const double *Kc, double *u, int *iters, double *w, hipStream_t st)
 {
-  if (dim == 2)
-    hipLaunchKernelGGL(mg_small_kernel<2>, dim3(1), dim3(kTailThreads), 0, st, g, Kc, u, iters, w);
-  else
-    hipLaunchKernelGGL(mg_small_kernel<3>, dim3(1), dim3(kTailThreads), 0, st, g, Kc, u, iters, w);
+  hipLaunchKernelGGL(mg_small_kernel<2>, dim3(1), dim3(kTailThreads), 0, st, g, Kc, u, iters, w);
   return hipGetLastError();
 }
 

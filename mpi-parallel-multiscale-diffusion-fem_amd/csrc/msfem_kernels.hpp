@@ -157,11 +157,11 @@ struct MgState {
 MgLayout mg_layout(int dim, int nc);
 // Galerkin levels, x = Dirichlet values, residual, state; then blocks of an even number of
 // iterations until the state says done (iterations past that end at once).  The solution is at
-// w + off_cx.  launch_mg_small: the whole iteration of a system with g.tail == 0.
+// w + off_cx.  launch_mg_small: the whole iteration of a 2D system with g.tail == 0.
 hipError_t launch_mg_setup(int dim, const MgLayout &g, const double *Kc, const double *Fc, const unsigned char *cmask,
                            const double *cval, double rel_tol, int max_iter, double *w, hipStream_t st);
 hipError_t launch_mg_iterations(int dim, const MgLayout &g, int count, const double *Kc, double *w, hipStream_t st);
-hipError_t launch_mg_small(int dim, const MgLayout &g, const double *Kc, double *u, int *iters, double *w, hipStream_t st);
+hipError_t launch_mg_small(const MgLayout &g, const double *Kc, double *u, int *iters, double *w, hipStream_t st);
 
 // coarse.hip
 hipError_t launch_coarse_assemble(int dim, int nc, const double *Ae, const double *Fe, int bc_kind, double *Kc,
