@@ -31,7 +31,10 @@ reference's default MatrixCoeff problem), quad64 (64^2 general quadrilaterals).
 Algorithmic work per CG iteration of a problem with N_I interior nodes:
 F_iter = (2*3^d - 1 + 10) N_I flops (stencil + CG vector updates), plus
 8 N_I + 2*49^2 for the two-level correction where it runs, plus f_ml(nf)
-(75 496 at 64^2) for the intermediate hat levels where they run.  The CPU
+(75 496 at 64^2) for the intermediate hat levels where they run.  Cells that
+the direct local solve took (one or two passes reported as iterations) count
+f_direct(nf) flops a pass instead: the eliminations of one nested dissection.
+The CPU
 baseline is the oracle's restatement of the reference's own recipe (CG +
 SSOR(1.6), absolute tolerance 1e-12, 1000 iterations;
 include/base/diffusion_problem_basis.tpp:295-317) on a sample of the same
@@ -58,7 +61,7 @@ PEAK_BF16_MFMA_TFLOPS = 2500.0  # dense
 # WRITE_SIZE passes scaled by a plain copy of known size (--copy-calibration):
 # profiles/local_solve_2d_lognormal64_hbm_traffic.md (FP64, 4096 cells) and
 # profiles/local_solve_2d_fp32_grf128_hbm_traffic.md (FP32 energy rule, 16384 cells)
-TRAFFIC_BYTES = {("lognormal64", 0): 2.946802e9, ("surrogate128", 1): 9.696504e9}
+TRAFFIC_BYTES = {("surrogate128", 1): 9.696504e9}
 METRIC = "coarse-cell bases built/sec: plain FP64 vs batched FP32+surrogate @1e-6 err"
 TAU = 5e-7  # energy stopping rule of the FP32 legs: a 2x margin on the 1e-6 relative energy-norm bar
 WEIGHTS = os.path.join(PKG, "surrogate_weights.npz")
@@ -79,6 +82,23 @@ def f_ml(nf):
         f += m * n * 2 * (2 * s - 1) + m * m * 2 * (2 * s - 1)  # restriction
         f += m * m                                               # D_s^-1
         f += m * n * 3 + n * n * 3                               # prolongation
+    return f
+
+
+def f_direct(nf):
+    """Algorithmic flops of one direct solve of a 2D cell with its four right-hand
+    sides: per block (side s; halved until at most 8) the elimination of its inner
+    lines' nodes, or a leaf's interior, from a symmetric front that holds them, the
+    block's outline and four rows more."""
+    levels = 1
+    while (8 << levels) < nf:
+        levels += 1
+    f = 0.0
+    for level in range(levels + 1):
+        s = nf / 2 ** level
+        e = 2 * s - 3 if level < levels else (s - 1) ** 2
+        m = e + (4 * s if level else 0) + 4
+        f += 4 ** level * (m ** 3 - (m - e) ** 3) / 3
     return f
 
 
@@ -417,7 +437,11 @@ def bench_workload(args):
     w = 8 if main_prec == msfem.PREC_FP64 else 4
     stride = msfem.coef_stride(dim, case["coef_kind"])
     b_iter = 11 * (nf_arr + 1) ** dim * w + nf_arr ** dim * stride * w   # per cell
-    flops = float((its.sum(axis=1) * f_iter).sum())
+    direct = (its.max(axis=1) <= 2) & (dim == 2)
+    work = its.sum(axis=1) * f_iter
+    work = np.where(direct, its.max(axis=1) * np.array([f_direct(int(k)) for k in nf_arr]), work)
+    flops = float(work.sum())
+    solver = "direct" if direct.all() else "CG" if not direct.any() else "direct and CG"
     peak = PEAK_FP64_TFLOPS if main_prec == msfem.PREC_FP64 else PEAK_FP32_TFLOPS
     achieved = flops / (solve_ms * 1e-3) / 1e12
     b_cell = nf_arr ** dim * stride * 8 + nb * (nf_arr + 1) ** dim * 8 + (nb * nb + nb) * 8
@@ -441,13 +465,15 @@ def bench_workload(args):
         "config": {"workload": f"{args.workload}: {desc}", "coarse_cells": n, "dim": dim,
                    "fine_per_cell": classes, "local_solves": n * nb, "path": pname[main_prec],
                    "autotuned_classes": tuned, "launch": "HIP graph, one concurrent branch per size class",
+                   "direct_cells": int(direct.sum()),
                    "two_level_cells": int((cs > 0).sum()), "intermediate_level_cells": int((cs == 2).sum())},
-        "roofline": {"bound": "mfma", "engine": "valu", "kernel": f"local_solve_{dim}d ({pname[main_prec]} CG)",
+        "roofline": {"bound": "mfma", "engine": "valu", "kernel": f"local solves ({pname[main_prec]}, {solver})",
                      "achieved": round(achieved, 3), "peak": peak, "unit": "TFLOP/s",
-                     "frac": round(achieved / peak, 4), "traffic": TRAFFIC_BYTES.get((args.workload, main_prec)),
+                     "frac": round(achieved / peak, 4), "traffic": None if direct.any() else TRAFFIC_BYTES.get((args.workload, main_prec)),
                      "kernel_ms": round(solve_ms, 4),
                      "flops_per_launch": flops,
-                     "lds_model_TBps": round(float((its.sum(axis=1) * b_iter).sum()) / (solve_ms * 1e-3) / 1e12, 2),
+                     "lds_model_TBps": None if direct.any() else
+                     round(float((its.sum(axis=1) * b_iter).sum()) / (solve_ms * 1e-3) / 1e12, 2),
                      "hbm_GBps": round(float(b_cell.sum()) / (ms * 1e-3) / 1e9, 2)},
         "iterations": {pname[p] + "_mean": round(float(r["its"].mean()), 1) for p, r in res.items()},
         "variants": {pname[p] + "_solve_kernel_ms": round(r["solve_kernel_ms"], 4) for p, r in res.items()},
